@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "../../include/metalllm_attn.h"
 
@@ -46,7 +47,13 @@ __global__ void __launch_bounds__(256) cast_kernel(const float* __restrict__ in,
 unsigned grid_for(size_t items) { return (unsigned)std::max<size_t>(1, std::min<size_t>((items + 255) / 256, 8192)); }
 
 __device__ __forceinline__ float bf_f(uint32_t h) { return __uint_as_float(h << 16); }
-__device__ __forceinline__ float bf_round(float f) { return bf_f(to_bf16(f)); }
+// Two floats -> packed bf16 pair by v_cvt_pk_bf16_f32: to_bf16's result for every float, NaNs
+// included (compared over all 2^32 of them).
+__device__ __forceinline__ uint32_t pk_bf16(float lo, float hi) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{lo, hi}, b2));
+}
 
 // out = bf16(a + b), eight elements per thread and step
 __global__ void __launch_bounds__(256) residual_kernel(const uint4* __restrict__ a, const uint4* __restrict__ b,
@@ -71,10 +78,25 @@ __global__ void __launch_bounds__(256) residual_kernel(const uint4* __restrict__
   }
 }
 
-// Sum over the 64 lanes of a wave, the same result in every lane.
+// Sum over the 64 lanes of a wave, the same result in every lane: the butterfly over partners at
+// distance 32, 16, 8, 4, 2, 1 in register moves (no LDS permutes, whose latency a row's two sums
+// would wait for six times). After the first three levels the lanes i and i ^ 8 hold the same
+// value, so a rotation by 4 within the row of 16 reaches the partner i ^ 4.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+  const uint32_t u = __float_as_uint(v);
+  auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const uint32_t w = __float_as_uint(v);
+  auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+  v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  v += dpp<0x128>(v);  // row_ror:8
+  v += dpp<0x124>(v);  // row_ror:4
+  v += dpp<0x4e>(v);   // quad_perm 2,3,0,1
+  v += dpp<0xb1>(v);   // quad_perm 1,0,3,2
   return v;
 }
 
@@ -98,15 +120,19 @@ __device__ __forceinline__ void unpack8(const uint4& u, float (&f)[8]) {
   const uint32_t w[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    f[2 * k] = bf_f(w[k] & 0xffffu);
-    f[2 * k + 1] = bf_f(w[k] >> 16);
+    f[2 * k] = __uint_as_float(w[k] << 16);
+    f[2 * k + 1] = __uint_as_float(w[k] & 0xffff0000u);
   }
 }
 __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
   uint32_t w[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) w[k] = to_bf16(f[2 * k]) | (to_bf16(f[2 * k + 1]) << 16);
+  for (int k = 0; k < 4; ++k) w[k] = pk_bf16(f[2 * k], f[2 * k + 1]);
   return uint4{w[0], w[1], w[2], w[3]};
+}
+// rounds eight floats in place to bf16 values
+__device__ __forceinline__ void round8(float (&f)[8]) {
+  unpack8(pack8(f), f);
 }
 
 // layernorm.metal:10-70, one row per wave, four waves per workgroup.
@@ -165,80 +191,179 @@ __global__ void __launch_bounds__(256) ln_fwd_kernel(const uint16_t* __restrict_
   }
 }
 
-// layernorm.metal:73-127. Wave w of workgroup g handles rows g*4 + w, then + 4*gridDim.x, ...;
-// each lane keeps the dgamma/dbeta partial sums of its own columns across those rows; the four
-// waves' partials meet in LDS and one fp32 atomic per column adds the workgroup's sum.
-template <int NCH>
-__global__ void __launch_bounds__(256) ln_bwd_kernel(uint16_t* __restrict__ dZ, const uint16_t* __restrict__ xnorm,
-                                                     const uint16_t* __restrict__ gamma,
-                                                     const float* __restrict__ stdev, uint16_t* __restrict__ dxnorm,
-                                                     float* __restrict__ dgamma, float* __restrict__ dbeta,
-                                                     uint32_t rows, uint32_t cols) {
-  __shared__ float red[2][4][64 * NCH * 8];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// layernorm.metal:73-127. A workgroup of 16 waves takes 16/S rows at a time, each by S waves (S > 1
+// for rows of more than 1024 columns, so that a lane holds at most two 16-byte chunks of a row: with
+// whole wide rows per lane the sums and the row leave room for one wave per SIMD). Row r of the
+// workgroup's k-th step is (k*gridDim.x + blockIdx.x)*16/S + r. Each lane keeps the dgamma/dbeta
+// partial sums of its own columns across its rows; the waves' partials meet in LDS and one fp32
+// atomic per column adds the workgroup's sum. All workgroups add into the same 2*cols addresses and
+// atomics on one address run one after another (about 34 ns each), so the grid is a compromise
+// (ln_bwd_grid). Four waves a workgroup, up to 1024 workgroups, rounding in integer arithmetic and
+// row sums through LDS permutes took 48 us at 16384 x 768, 71 us at 32768 x 1024 and 85 us at 4096 x
+// 4096; this takes 24, 35 (5.8 TB/s) and 24 us.
+// BLOCK (the phase encoder's form): the gradient comes in as the fp32 dX and is rounded to bf16
+// first (castFloatToBfloat), and `add` is added to the result, rounded again (residualAdd): the
+// three kernels' results bit for bit, with one read of dX and one write of dZ instead of three and
+// two passes over the rows.
+template <int NC, int S, bool BLOCK>
+__global__ void __launch_bounds__(1024) ln_bwd_kernel(uint16_t* __restrict__ dZ, const float* __restrict__ dX,
+                                                      const uint16_t* __restrict__ add,
+                                                      const uint16_t* __restrict__ xnorm,
+                                                      const uint16_t* __restrict__ gamma,
+                                                      const float* __restrict__ stdev, uint16_t* __restrict__ dxnorm,
+                                                      float* __restrict__ dgamma, float* __restrict__ dbeta,
+                                                      uint32_t rows, uint32_t cols) {
+  constexpr int W = 16, RW = W / S;  // waves, rows per step
+  __shared__ float red[2][W][512];
+  __shared__ float2 rsum[2][W];  // S > 1: the waves' parts of a row's two sums, by step parity
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rg = wave / S, sub = wave % S;
   const int nchunk = (int)(cols / 8);
-  float pg[NCH][8], pb[NCH][8];
+  const int c0 = lane + 64 * NC * sub;  // this lane's first 16-byte chunk of a row
+  float pg[NC][8], pb[NC][8];
+  uint4 gam[NC];
 #pragma unroll
-  for (int j = 0; j < NCH; ++j)
+  for (int j = 0; j < NC; ++j) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) pg[j][k] = pb[j][k] = 0.0f;
-  for (uint32_t row = blockIdx.x * 4 + wave; row < rows; row += 4 * gridDim.x) {
-    const size_t base = (size_t)row * cols;
-    RowChunks<NCH> dz, xn;
-    load_row<NCH>((const uint4*)(dZ + base), nchunk, lane, dz);
-    load_row<NCH>((const uint4*)(xnorm + base), nchunk, lane, xn);
-    float dxn[NCH][8];
+    const int c = c0 + 64 * j;
+    gam[j] = c < nchunk ? ((const uint4*)gamma)[c] : uint4{0u, 0u, 0u, 0u};
+  }
+  const uint4 none = uint4{0u, 0u, 0u, 0u};
+  for (uint32_t r0 = blockIdx.x * RW, it = 0; r0 < rows; r0 += RW * gridDim.x, ++it) {
+    const uint32_t row = r0 + rg;
+    const bool live = row < rows;  // false only past the last row: the wave adds zeros and stores nothing
+    const size_t base = (size_t)min(row, rows - 1) * cols;
+    uint4 dz[NC], xn[NC], ad[BLOCK ? NC : 1], dxn[NC];
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      // chunks past the row are read in bounds and taken as zeros: loads behind a per-lane branch
+      // are waited for one by one (32768 x 1024: 43 us, 35 us without the branch)
+      const bool in = live && c0 + 64 * j < nchunk;
+      const int c = min(c0 + 64 * j, nchunk - 1);
+      const uint4 x = ((const uint4*)(xnorm + base))[c];
+      xn[j] = in ? x : none;
+      if constexpr (BLOCK) {
+        const uint4 a = ((const uint4*)(dX + base))[2 * c], b = ((const uint4*)(dX + base))[2 * c + 1];
+        ad[j] = ((const uint4*)(add + base))[c];
+        dz[j] = uint4{pk_bf16(__uint_as_float(a.x), __uint_as_float(a.y)), pk_bf16(__uint_as_float(a.z), __uint_as_float(a.w)),
+                      pk_bf16(__uint_as_float(b.x), __uint_as_float(b.y)), pk_bf16(__uint_as_float(b.z), __uint_as_float(b.w))};
+      } else {
+        dz[j] = ((const uint4*)(dZ + base))[c];
+      }
+      if (!in) dz[j] = none;
+    }
+    const float rdev = 1.0f / stdev[min(row, rows - 1)];
     float s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NCH; ++j) {
-      const int c = lane + 64 * j;
-      float z[8], x[8], g[8];
-      unpack8(dz.v[j], z);
-      unpack8(xn.v[j], x);
-      if (c < nchunk) unpack8(((const uint4*)gamma)[c], g);
-      else
-#pragma unroll
-        for (int k = 0; k < 8; ++k) g[k] = 0.0f;
+    for (int j = 0; j < NC; ++j) {
+      float z[8], x[8], g[8], a[8], d[8], t[8];
+      unpack8(dz[j], z);
+      unpack8(xn[j], x);
+      // opaque: gamma stays packed across rows (hoisted, its floats take the registers of a row)
+      asm volatile("" : "+v"(gam[j].x), "+v"(gam[j].y), "+v"(gam[j].z), "+v"(gam[j].w));
+      unpack8(gam[j], g);
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        pg[j][k] += bf_round(x[k] * z[k]);  // bfloat * bfloat is a bfloat
-        pb[j][k] += z[k];
-        dxn[j][k] = bf_round(z[k] * g[k]);
-        s1 += dxn[j][k];
-        s2 += bf_round(dxn[j][k] * x[k]);
+        a[k] = x[k] * z[k];
+        d[k] = z[k] * g[k];
       }
-      if (dxnorm && c < nchunk) ((uint4*)(dxnorm + base))[c] = pack8(dxn[j]);
+      round8(a);  // bfloat * bfloat is a bfloat
+      dxn[j] = pack8(d);
+      unpack8(dxn[j], d);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) t[k] = d[k] * x[k];
+      round8(t);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        pg[j][k] += a[k];
+        pb[j][k] += z[k];
+        s1 += d[k];
+        s2 += t[k];
+      }
+      const int c = c0 + 64 * j;
+      if (!BLOCK && dxnorm && live && c < nchunk) ((uint4*)(dxnorm + base))[c] = dxn[j];
     }
-    const float rs1 = wave_sum(s1) / (float)cols;
-    const float rs2 = wave_sum(s2) / (float)cols;
-    const float rdev = 1.0f / stdev[row];
+    s1 = wave_sum(s1);
+    s2 = wave_sum(s2);
+    if constexpr (S > 1) {
+      if (lane == 0) rsum[it & 1][wave] = float2{s1, s2};
+      __syncthreads();  // the other parity's slots were read before the previous step's barrier
+      s1 = s2 = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NCH; ++j) {
-      const int c = lane + 64 * j;
-      if (c >= nchunk) continue;
-      float x[8], o[8];
-      unpack8(xn.v[j], x);
+      for (int u = 0; u < S; ++u) {
+        const float2 v = rsum[it & 1][rg * S + u];
+        s1 += v.x;
+        s2 += v.y;
+      }
+    }
+    const float rs1 = s1 / (float)cols, rs2 = s2 / (float)cols;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) o[k] = rdev * ((dxn[j][k] - rs1) - x[k] * rs2);
+    for (int j = 0; j < NC; ++j) {
+      const int c = c0 + 64 * j;
+      if (!live || c >= nchunk) continue;
+      float x[8], d[8], o[8];
+      unpack8(xn[j], x);
+      unpack8(dxn[j], d);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) o[k] = rdev * ((d[k] - rs1) - x[k] * rs2);
+      if constexpr (BLOCK) {
+        float r[8];
+        unpack8(ad[j], r);
+        round8(o);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) o[k] += r[k];
+      }
       ((uint4*)(dZ + base))[c] = pack8(o);
     }
   }
-  // column partials of the four waves -> one atomic per column
+  // column partials of the waves that share columns -> one atomic per column
 #pragma unroll
-  for (int j = 0; j < NCH; ++j)
+  for (int j = 0; j < NC; ++j) {
+    if (j) __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int col = 8 * (lane + 64 * j) + k;
-      red[0][wave][col] = pg[j][k];
-      red[1][wave][col] = pb[j][k];
+    for (int k = 0; k < 8; k += 4) {
+      *(float4*)&red[0][wave][8 * lane + k] = float4{pg[j][k], pg[j][k + 1], pg[j][k + 2], pg[j][k + 3]};
+      *(float4*)&red[1][wave][8 * lane + k] = float4{pb[j][k], pb[j][k + 1], pb[j][k + 2], pb[j][k + 3]};
     }
-  __syncthreads();
-  for (uint32_t col = threadIdx.x; col < cols; col += 256) {
-    const float g = red[0][0][col] + red[0][1][col] + red[0][2][col] + red[0][3][col];
-    const float b = red[1][0][col] + red[1][1][col] + red[1][2][col] + red[1][3][col];
-    atomicAdd(dgamma + col, g);
-    atomicAdd(dbeta + col, b);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < 1024 * S; i += 1024) {
+      const uint32_t which = (i >> 9) & 1, u = i >> 10, c = i & 511, col = 512 * (NC * u + j) + c;
+      if (col >= cols) continue;
+      float sum = red[which][u][c];
+#pragma unroll
+      for (int w = 1; w < RW; ++w) sum += red[which][w * S + u][c];
+      atomicAdd((which ? dbeta : dgamma) + col, sum);
+    }
   }
+}
+
+// Workgroups of ln_bwd_kernel: the rows' traffic (6 bytes an element, about 20 GB/s a workgroup)
+// takes t = 6 rows cols / (20e9 n) seconds on n of them and the atomics 34e-9 n; the sum is least at
+// n = 0.094 sqrt(rows cols), and there is one workgroup per CU.
+uint32_t ln_bwd_grid(uint32_t rows, uint32_t cols, int rows_per_step) {
+  const uint32_t n = (uint32_t)(0.094 * std::sqrt((double)rows * cols));
+  const uint32_t steps = (rows + rows_per_step - 1) / rows_per_step;
+  return std::max<uint32_t>(1, std::min<uint32_t>(steps, std::min<uint32_t>(256, std::max<uint32_t>(n, 16))));
+}
+
+template <bool BLOCK>
+hipError_t launch_ln_bwd(uint16_t* dZ, const float* dX, const uint16_t* add, const uint16_t* xnorm, const uint16_t* gamma,
+                         const float* stdev, uint16_t* dxnorm, float* dgamma, float* dbeta, uint32_t rows, uint32_t cols,
+                         hipStream_t s) {
+  const int nch = (int)((cols / 8 + 63) / 64);
+  const int S = nch <= 2 ? 1 : (nch <= 4 ? 2 : 4);
+  const dim3 grid(ln_bwd_grid(rows, cols, 16 / S));
+#define LNB(NC, S_) \
+  hipLaunchKernelGGL((ln_bwd_kernel<NC, S_, BLOCK>), grid, dim3(1024), 0, s, dZ, dX, add, xnorm, gamma, stdev, dxnorm, \
+                     dgamma, dbeta, rows, cols)
+  if (nch == 1) LNB(1, 1);
+  else if (S == 1) LNB(2, 1);
+  else if (S == 2) LNB(2, 2);
+  else LNB(2, 4);
+#undef LNB
+  return hipGetLastError();
 }
 
 int validate_ln(const LayernormParams* p) {
@@ -252,6 +377,16 @@ int validate_ln(const LayernormParams* p) {
 bool al16(const void* q) { return ((uintptr_t)q & 15u) == 0; }
 
 }  // namespace
+
+namespace mla {
+// The phase encoder's end of the backward (model.h:692-695) in one launch: dStream =
+// bf16(ln backward(bf16(dX)) + dOut), dgamma and dbeta added into.
+hipError_t launch_block_ln_bwd(const float* dX, const uint16_t* dOut, const uint16_t* xnorm, const uint16_t* gamma,
+                               const float* stdev, uint16_t* dStream, float* dgamma, float* dbeta, uint32_t rows,
+                               uint32_t cols, hipStream_t s) {
+  return launch_ln_bwd<true>(dStream, dX, dOut, xnorm, gamma, stdev, nullptr, dgamma, dbeta, rows, cols, s);
+}
+}  // namespace mla
 
 extern "C" {
 
@@ -298,23 +433,10 @@ int layernormBackward(uint16_t* dZ, const uint16_t* x_norm_cache, const uint16_t
   if (!al16(dZ) || !al16(x_norm_cache) || !al16(gamma) || !al16(stdev) || !al16(dgamma) || !al16(dbeta) ||
       (dx_norm && !al16(dx_norm)))
     return METALLLM_ATTN_E_ALIGN;
-  // enough workgroups to fill the chip, each summing its columns over many rows
-  const dim3 grid(std::min<uint32_t>((p->rows + 3) / 4, 1024));
-  const hipStream_t s = (hipStream_t)stream;
-  const int nch = (int)((p->cols / 8 + 63) / 64);
-#define LNB(N) hipLaunchKernelGGL(ln_bwd_kernel<N>, grid, dim3(256), 0, s, dZ, x_norm_cache, gamma, stdev, dx_norm, dgamma, dbeta, p->rows, p->cols)
-  switch (nch) {
-    case 1: LNB(1); break;
-    case 2: LNB(2); break;
-    case 3: LNB(3); break;
-    case 4: LNB(4); break;
-    case 5: LNB(5); break;
-    case 6: LNB(6); break;
-    case 7: LNB(7); break;
-    default: LNB(8); break;
-  }
-#undef LNB
-  return hipGetLastError() == hipSuccess ? METALLLM_ATTN_OK : METALLLM_ATTN_E_LAUNCH;
+  return launch_ln_bwd<false>(dZ, nullptr, nullptr, x_norm_cache, gamma, stdev, dx_norm, dgamma, dbeta, p->rows, p->cols,
+                              (hipStream_t)stream) == hipSuccess
+             ? METALLLM_ATTN_OK
+             : METALLLM_ATTN_E_LAUNCH;
 }
 
 int castFloatToBfloat(const float* in, uint16_t* out, uint32_t count, metalllm_stream_t stream) {

@@ -33,6 +33,12 @@ namespace mla {  // attn_fwd.hip
 void forward_prepare();
 }  // namespace mla
 
+namespace mla {  // glue.hip
+hipError_t launch_block_ln_bwd(const float* dX, const uint16_t* dOut, const uint16_t* xnorm, const uint16_t* gamma,
+                               const float* stdev, uint16_t* dStream, float* dgamma, float* dbeta, uint32_t rows,
+                               uint32_t cols, hipStream_t s);
+}  // namespace mla
+
 namespace mla {  // sublayer_gemm.hip
 bool grad_dx_fused_ok(int R, int C);
 hipError_t launch_grad_dx(float* dX, const float* dQ, const uint16_t* dK, const uint16_t* dV, const uint16_t* Wq,
@@ -585,12 +591,11 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
     TRY(op_grad_dw(c, b->X, b->dQ, split, lo, b->dK, b->dV, b->dQw, b->dKw, b->dVw, R, C, partial, false));
   }
   if (c.query) return METALLLM_ATTN_OK;
-  if (block) {  // model.h:692-695
-    TRY(castFloatToBfloat(b->dX, b->dStream, (uint32_t)e, s));
-    TRY(layernormBackward(b->dStream, b->ln_xnorm, b->ln_gamma, b->ln_stdev, nullptr, b->ln_dgamma, b->ln_dbeta, &lp,
-                          s));
-    return residualAdd(b->dStream, b->dOut, b->dStream, (uint32_t)e, s);
-  }
+  if (block)  // model.h:692-695: cast of dX, ln1 backward and the skip add
+    return mla::launch_block_ln_bwd(b->dX, b->dOut, b->ln_xnorm, b->ln_gamma, b->ln_stdev, b->dStream, b->ln_dgamma,
+                                    b->ln_dbeta, (uint32_t)R, (uint32_t)C, c.stream) == hipSuccess
+               ? METALLLM_ATTN_OK
+               : METALLLM_ATTN_E_LAUNCH;
   if (b->dX_bf16) TRY(castFloatToBfloat(b->dX, b->dX_bf16, (uint32_t)e, s));
   return METALLLM_ATTN_OK;
 }

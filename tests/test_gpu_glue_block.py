@@ -1,0 +1,41 @@
+"""layernormBackward where a row is shared by one, two and four waves, with row counts that leave the
+last step of a workgroup partly empty, against the oracle at the bars of test_gpu_glue.py; and the
+phase encoder's form (dX cast, ln1 backward and skip add in one kernel) bit for bit against the
+three public calls on the encoder's own dX."""
+import numpy as np
+import pytest
+
+import oracle as O
+from tests import test_gpu_glue as glue_checks
+from tests.attn_case import to_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,cols", [(4099, 1032), (1000, 1536), (515, 2056), (33, 3080), (1, 1024), (17, 512)])
+def test_layernorm_row_split(gpu, rows, cols):
+    import metalllm_amd.glue as G
+    glue_checks.test_layernorm_forward_backward(gpu, G, rows, cols, 1.0)
+
+
+@pytest.mark.parametrize("B,T,H,C", [(1, 64, 1, 64), (3, 192, 6, 384), (2, 64, 12, 768), (1, 128, 20, 1280), (1, 64, 20, 2560)])
+def test_block_backward_end(gpu, B, T, H, C):
+    import torch
+    import metalllm_amd.glue as G
+    import metalllm_amd.sublayer as S
+    rng = np.random.default_rng(B * T + C)
+    bf = lambda shape, sc=1.0, sh=0.0: to_gpu(O.f32_to_bf16((rng.standard_normal(shape) * sc + sh).astype(np.float32)), gpu)
+    blk = S.Sublayer(None, *[bf((C, C), 0.02) for _ in range(4)], H=H, hidden=bf((B, T, C), 1.0, 0.3),
+                     ln_gamma=bf((C,), 0.1, 1.0), ln_beta=bf((C,), 0.1))
+    blk.dOut.copy_(bf((B, T, C)))
+    blk.encode(0)
+    blk.encode(1)
+    d = torch.empty_like(blk.dOut)
+    dg, db = torch.zeros(C, device=gpu), torch.zeros(C, device=gpu)
+    G.castFloatToBfloat(blk.dX, d)
+    G.layernormBackward(d, blk.ln_xnorm, blk.ln_gamma, blk.ln_stdev, dg, db)
+    G.residualAdd(d, blk.dOut, d)
+    torch.cuda.synchronize()
+    assert torch.equal(d, blk.dStream)
+    for a, b in ((blk.ln_dgamma, dg), (blk.ln_dbeta, db)):  # fp32 column sums in atomic order
+        assert (a - b).abs().max().item() <= 1e-5 * b.abs().max().item()
