@@ -112,20 +112,39 @@ __host__ __device__ inline void decode_workgroup(int bid, int npairs, int nblk, 
   blk = last_first ? (nblk - 1 - local) : local;
 }
 
+// Workgroups are dealt to the XCDs in turn and, inside an XCD, to its CUs in turn while they are
+// free: ids that differ by a multiple of kCus start on the same CU.
+constexpr int kCus = 256;
+
 // Item k of workgroup `bid` of a persistent grid of `grid` workgroups over npairs x nblk
 // (pair, block) items; false when the workgroup has fewer than k + 1 items. When both the pair
 // count and the grid are multiples of 8, the workgroups on XCD x (bid % 8 == x) serve the pairs
 // p = x (mod 8), so all blocks of a pair share one L2; otherwise all workgroups form one group.
-// A group's items are listed pair by pair, each pair's last (largest causal) block first, and
-// dealt in snake order over its workgroups, so each workgroup gets about the same work.
+// With two items or more per workgroup a group's items are listed pair by pair, each pair's last
+// (largest causal) block first, and dealt in snake order over its workgroups: every workgroup gets
+// about the same work, and the workgroups running at once share a few pairs' tiles in L2. With fewer
+// the list goes block by block, longest first, and its first W items snake over rows of one
+// workgroup per CU, so that the workgroups that share a CU have about the same work together. (Pair
+// by pair, the workgroups w, w + 256 and w + 512 of 12 pairs of T = 8192 all had blocks of the same
+// length and the CUs with the longest three took twice the mean: 204 us.)
 __host__ __device__ inline bool fwd_item_of(int bid, int grid, int k, int npairs, int nblk, int& pair, int& blk) {
   const int G = ((npairs & 7) == 0 && (grid & 7) == 0) ? 8 : 1;
-  const int x = bid % G, w = bid / G, W = grid / G;
+  const int x = bid % G, W = grid / G, n = npairs / G * nblk;
+  int w = bid / G;
+  const bool few = n < 2 * W;
+  if (few) {
+    const int row = kCus / G, r = w / row;
+    if (r & 1) {  // this row's ids in reverse
+      const int end = (r + 1) * row < W ? (r + 1) * row : W;
+      w = r * row + (end - 1 - w);
+    }
+  }
   const int m = k * W + ((k & 1) ? W - 1 - w : w);
-  if (m >= npairs / G * nblk) return false;
-  const int j = m / nblk, local = m - j * nblk;
-  pair = j * G + x;
-  blk = nblk - 1 - local;
+  if (m >= n) return false;
+  const int per = few ? npairs / G : nblk;
+  const int i = m / per, j = m - i * per;
+  pair = (few ? j : i) * G + x;
+  blk = nblk - 1 - (few ? i : j);
   return true;
 }
 
