@@ -87,10 +87,10 @@ int computeD(const uint16_t* dO, const uint16_t* O, float* D, const AttentionPar
 /* Replaces the flashAttentionBackward dispatch at model.h:648-665 (attention.metal:198-299).
  * dZ is dO; d and l are computeD's and the forward's outputs. dQ += gradient (fp32, accumulated
  * into as in the reference: zero it first for the plain gradient); dK, dV = gradients (bf16).
- * Two kernels: dK/dV by key-block owners, then dQ by query-block owners, each recomputing the
- * softmax tile it needs. For D = 64 and M <= 256 (the reference's own shape) one kernel does
- * both: a workgroup per (b, head) keeps the dS tiles in LDS (dK, dV bit-identical to the
- * two-kernel path). */
+ * One launch: dK/dV by key-block owners and dQ by query-block owners, each recomputing the
+ * softmax tile it needs. For D = 64 and M = 256 (the reference's own shape), where B*NH fills whole
+ * rounds of one pair per CU, a workgroup per (b, head) does both and keeps the dS tiles in LDS (dK,
+ * dV bit-identical to the other form's, dQ equal up to fp32 summation order). */
 int flashAttentionBackward(const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
                            const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
                            const AttentionParams* p, metalllm_stream_t stream);
@@ -111,11 +111,11 @@ int metalllmAttnBackwardWorkspaceSize(const AttentionParams* p, uint64_t* bytes)
  * what flashAttentionBackward adds into a zeroed dQ up to fp32 summation order. The workspace
  * holds no state between calls, but one
  * workspace must not serve two calls at once. Returns METALLLM_ATTN_E_NULL / _E_ALIGN / _E_SIZE
- * for a NULL, misaligned or too small workspace. At D = 64 no dS is stored and the workspace is
- * validated but not used: for M <= 256 it runs the same single kernel as flashAttentionBackward
- * there (dS stays in LDS); for longer sequences flashAttentionBackward's two kernels, the dQ kernel
- * writing dQ instead of adding into it (at this head size the recomputation is faster than the dS
- * round trip), so dQ, dK and dV equal flashAttentionBackward's into a zeroed dQ bit for bit.
+ * for a NULL, misaligned or too small workspace. At D = 64, and at D = 128 while B*NH*ceil(M/128) is
+ * at most 512 (two workgroups per CU), no dS is stored and the workspace is validated but not used:
+ * it runs flashAttentionBackward's kernel writing dQ instead of adding into it (there the
+ * recomputation in one launch is faster than the dS round trip's two), so dQ, dK and dV equal
+ * flashAttentionBackward's into a zeroed dQ bit for bit.
  * No counterpart in the reference. */
 int flashAttentionBackwardWorkspace(const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
                                     const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
@@ -310,13 +310,14 @@ int metalllmSublayerGraphDestroy(metalllmSublayerGraph* g);
 
 /* Bench hook (no counterpart in the reference): launches one of the kernels of the two backward
  * entry points on `stream`: part 0 = dK/dV and part 1 = dQ recomputing the softmax
- * (flashAttentionBackward is exactly part 0 then part 1); part 2 = dK/dV storing dS into the
- * workspace and part 3 = dQ from the stored dS (flashAttentionBackwardWorkspace is exactly part 2
- * then part 3). Timing the parts separately measures the same work. Same validation and return
+ * (flashAttentionBackward does the work of part 0 and part 1, in one launch, bit for bit the same);
+ * part 2 = dK/dV storing dS into the workspace and part 3 = dQ from the stored dS
+ * (flashAttentionBackwardWorkspace: likewise part 2 and part 3, two launches where dS is stored). Same validation and return
  * codes as those entry points (parts 0 and 1 ignore the workspace arguments); a part outside
- * 0..3 returns METALLLM_ATTN_E_LAYOUT. For D = 64 and M <= 256 parts 0 and 2 launch the single
- * fused kernel (part 0 adds dQ, part 2 writes it) and parts 1 and 3 launch nothing. For D = 64 and
- * longer sequences parts 2 and 3 launch parts 0's and 1's kernels, part 3 writing dQ. */
+ * 0..3 returns METALLLM_ATTN_E_LAYOUT. Where the entry points run the fused short-sequence kernel,
+ * parts 0 and 2 launch it (part 0 adds dQ, part 2 writes it) and parts 1 and 3 launch nothing. Where
+ * the workspace entry point stores no dS, parts 2 and 3 launch parts 0's and 1's kernels, part 3
+ * writing dQ. */
 int metalllmAttnBackwardPart(int part, const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
                              const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
                              void* workspace, uint64_t workspace_bytes, const AttentionParams* p,

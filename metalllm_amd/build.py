@@ -16,7 +16,7 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "libmetalllm_attn.so")
-SOURCES = ["attn_abi.hip", "attn_fwd.hip", "attn_bwd.hip", "attn_bwd_dq.hip", "attn_bwd_dqs.hip", "attn_computed.hip",
+SOURCES = ["attn_abi.hip", "attn_fwd.hip", "attn_bwd.hip", "attn_bwd_dq.hip", "attn_bwd_both.hip", "attn_bwd_dqs.hip", "attn_computed.hip",
            "attn_noalloc.hip", "sublayer.hip", "sublayer_gemm.hip", "glue.hip"]
 LIBS = ["-L/opt/rocm/lib", "-lrocblas", "-Wl,-rpath,/opt/rocm/lib"]  # sublayer GEMMs
 
@@ -35,6 +35,7 @@ EXTRA = {
     "attn_fwd.hip": ["-mllvm", "-pragma-unroll-threshold=200000"],
     "attn_bwd.hip": ["-mllvm", "-pragma-unroll-threshold=200000"],
     "attn_bwd_dq.hip": ["-mllvm", "-pragma-unroll-threshold=200000"],
+    "attn_bwd_both.hip": ["-mllvm", "-pragma-unroll-threshold=200000"],
 }
 
 

@@ -21,6 +21,45 @@ bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 
 float head_scale(uint32_t D) { return 1.0f / std::sqrt((float)D); }  // attention.metal:109,268
 
+// One part of a backward entry point (metalllmAttnBackwardPart), or with `whole` the entry point
+// whose first part it is (0: flashAttentionBackward, 2: flashAttentionBackwardWorkspace).
+int backward(int part, const uint16_t* dZ, const float* d, const float* l, const uint16_t* q, const uint16_t* k,
+             const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV, void* workspace, uint64_t workspace_bytes,
+             const AttentionParams* p, metalllm_stream_t stream, bool whole) {
+  const int rc = validate(p);
+  if (rc) return rc;
+  if (part < 0 || part > 3) return METALLLM_ATTN_E_LAYOUT;
+  if (!dZ || !d || !l || !q || !k || !v || !dQ || !dK || !dV) return METALLLM_ATTN_E_NULL;
+  if (!aligned16(dZ) || !aligned16(d) || !aligned16(l) || !aligned16(q) || !aligned16(k) || !aligned16(v) ||
+      !aligned16(dQ) || !aligned16(dK) || !aligned16(dV))
+    return METALLLM_ATTN_E_ALIGN;
+  const int D = (int)p->D;
+  const hipStream_t s = (hipStream_t)stream;
+  mla::BwdArgs a{dZ, d, l, q, k, v, dQ, dK, dV, (int)p->M, (int)p->NH, (int)p->B, head_scale(p->D)};
+  const bool acc = part < 2;  // parts 0 and 1 add into dQ, 2 and 3 write it
+  if (!acc) {
+    if (!workspace) return METALLLM_ATTN_E_NULL;
+    if (!aligned16(workspace)) return METALLLM_ATTN_E_ALIGN;
+    if (workspace_bytes < (uint64_t)mla::ds_scratch_bytes(a.B, a.H, a.T)) return METALLLM_ATTN_E_SIZE;
+  }
+  const bool first = part == 0 || part == 2;
+  hipError_t e = hipSuccess;
+  if (mla::backward_is_short(a.T, D, a.B * a.H)) {
+    // one fused kernel computes dK, dV and dQ; the second part has nothing left to do
+    if (first) e = mla::launch_backward_short(a, acc, s);
+  } else if (acc || mla::workspace_recomputes(a.T, D, a.B * a.H)) {
+    e = whole   ? mla::launch_backward_both(a, D, acc, s)
+        : first ? mla::launch_backward(a, D, s)
+                : mla::launch_backward_dq(a, D, acc, s);
+  } else {
+    // dK/dV storing dS into the workspace, then dQ = dS.K
+    a.dS = (uint16_t*)workspace;
+    if (first) e = mla::launch_backward(a, D, s);
+    if (e == hipSuccess && (whole || !first)) e = mla::launch_backward_dqs(a, D, s);
+  }
+  return e == hipSuccess ? METALLLM_ATTN_OK : METALLLM_ATTN_E_LAUNCH;
+}
+
 }  // namespace
 
 extern "C" {
@@ -59,59 +98,20 @@ int metalllmAttnBackwardPart(int part, const uint16_t* dZ, const float* d, const
                              const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
                              void* workspace, uint64_t workspace_bytes, const AttentionParams* p,
                              metalllm_stream_t stream) {
-  const int rc = validate(p);
-  if (rc) return rc;
-  if (part < 0 || part > 3) return METALLLM_ATTN_E_LAYOUT;
-  if (!dZ || !d || !l || !q || !k || !v || !dQ || !dK || !dV) return METALLLM_ATTN_E_NULL;
-  if (!aligned16(dZ) || !aligned16(d) || !aligned16(l) || !aligned16(q) || !aligned16(k) || !aligned16(v) ||
-      !aligned16(dQ) || !aligned16(dK) || !aligned16(dV))
-    return METALLLM_ATTN_E_ALIGN;
-  mla::BwdArgs a{dZ, d, l, q, k, v, dQ, dK, dV, (int)p->M, (int)p->NH, (int)p->B, head_scale(p->D)};
-  if (part >= 2) {
-    if (!workspace) return METALLLM_ATTN_E_NULL;
-    if (!aligned16(workspace)) return METALLLM_ATTN_E_ALIGN;
-    if (workspace_bytes < (uint64_t)mla::ds_scratch_bytes(a.B, a.H, a.T)) return METALLLM_ATTN_E_SIZE;
-    a.dS = (uint16_t*)workspace;
-  }
-  if (mla::backward_is_short(a.T, (int)p->D)) {
-    // one fused kernel computes dK, dV and dQ (part 0 adds dQ, part 2 writes it); parts 1 and 3
-    // have nothing left to do
-    if (part == 1 || part == 3) return METALLLM_ATTN_OK;
-    return mla::launch_backward_short(a, part == 0, (hipStream_t)stream) == hipSuccess ? METALLLM_ATTN_OK
-                                                                                         : METALLLM_ATTN_E_LAUNCH;
-  }
-  hipError_t e;
-  if (part >= 2 && mla::workspace_recomputes(a.T, (int)p->D)) {
-    // the recomputing kernels, dQ written: faster than the dS round trip at this head size (the
-    // workspace is validated but not used)
-    a.dS = nullptr;
-    e = part == 2 ? mla::launch_backward(a, (int)p->D, (hipStream_t)stream)
-                  : mla::launch_backward_dq(a, (int)p->D, false, (hipStream_t)stream);
-  } else {
-    e = part == 0 || part == 2 ? mla::launch_backward(a, (int)p->D, (hipStream_t)stream)
-        : part == 1           ? mla::launch_backward_dq(a, (int)p->D, true, (hipStream_t)stream)
-                              : mla::launch_backward_dqs(a, (int)p->D, (hipStream_t)stream);
-  }
-  return e == hipSuccess ? METALLLM_ATTN_OK : METALLLM_ATTN_E_LAUNCH;
+  return backward(part, dZ, d, l, q, k, v, dQ, dK, dV, workspace, workspace_bytes, p, stream, false);
 }
 
 int flashAttentionBackward(const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
                            const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
                            const AttentionParams* p, metalllm_stream_t stream) {
-  // dK/dV by the key-block owners, then dQ by the query-block owners (both on `stream`, in order)
-  const int rc = metalllmAttnBackwardPart(0, dZ, d, l, q, k, v, dQ, dK, dV, nullptr, 0, p, stream);
-  if (rc) return rc;
-  return metalllmAttnBackwardPart(1, dZ, d, l, q, k, v, dQ, dK, dV, nullptr, 0, p, stream);
+  return backward(0, dZ, d, l, q, k, v, dQ, dK, dV, nullptr, 0, p, stream, true);
 }
 
 int flashAttentionBackwardWorkspace(const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
                                     const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
                                     void* workspace, uint64_t workspace_bytes, const AttentionParams* p,
                                     metalllm_stream_t stream) {
-  // dK/dV by the key-block owners, storing dS into the workspace; then dQ = dS.K
-  const int rc = metalllmAttnBackwardPart(2, dZ, d, l, q, k, v, dQ, dK, dV, workspace, workspace_bytes, p, stream);
-  if (rc) return rc;
-  return metalllmAttnBackwardPart(3, dZ, d, l, q, k, v, dQ, dK, dV, workspace, workspace_bytes, p, stream);
+  return backward(2, dZ, d, l, q, k, v, dQ, dK, dV, workspace, workspace_bytes, p, stream, true);
 }
 
 const char* metalllmAttnErrorString(int code) {

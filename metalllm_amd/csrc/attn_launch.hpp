@@ -55,15 +55,24 @@ hipError_t launch_backward(const BwdArgs& a, int D, hipStream_t s);     // dK, d
 // dQ (query-owner, recomputing dS): added into dQ (accumulate) or written
 hipError_t launch_backward_dq(const BwdArgs& a, int D, bool accumulate, hipStream_t s);
 hipError_t launch_backward_dqs(const BwdArgs& a, int D, hipStream_t s); // dQ from the stored dS
-// Short sequences (D = 64, T <= 256): dK, dV and dQ of a (b,h) pair by one workgroup, one launch,
-// no workspace; dQ added into (accumulate) or written.
-bool backward_is_short(int T, int D);
-// Whether the workspace entry point runs the recomputing kernels (dK/dV without the dS store, then
-// dQ written) instead of the dS round trip. Yes at D = 64: the dK/dV kernel without the store runs
-// three workgroups per CU and the pair is faster (config 2 step 0.436 -> 0.41 ms, config 4's
-// 0.733 -> 0.716 ms); T <= 256 runs the fused short backward instead (backward_is_short). No at
-// D = 128, where the round trip saves two of the seven products.
-inline bool workspace_recomputes(int T, int D) { return D == 64 && T > 256; }
+// launch_backward (without the dS store) and launch_backward_dq in one launch, the same results
+hipError_t launch_backward_both(const BwdArgs& a, int D, bool accumulate, hipStream_t s);
+// Sequences of four query tiles (D = 64, T = 256): dK, dV and dQ of a (b,h) pair by one workgroup
+// per CU, one launch, no workspace; dQ added into (accumulate) or written. It takes 21.5 us for
+// each round of kCus pairs, bwd_both_kernel 0.085-0.089 us a pair (and 10 us at least), so it is the
+// faster one only where its last round is nearly full: 768 pairs 63.6 against 64.7 us, 1536 pairs
+// 129.9 against 136.8, but 6 pairs 19.0 against 10.8, 320 pairs 42.5 against 30.5. At T <= 192 it is
+// nowhere faster by more than 1% (two tiles, 6 to 1536 pairs: 10.6-58.3 against 9.8-57.1 us).
+// Defined below, at kCus.
+__host__ __device__ inline bool backward_is_short(int T, int D, int pairs);
+// Whether the workspace entry point runs the recomputing kernels (dK/dV without the dS store and dQ
+// written, in one launch) instead of the dS round trip. Yes at D = 64: the dK/dV kernel without the
+// store runs three workgroups per CU and the pair is faster (config 2 step 0.436 -> 0.41 ms, config
+// 4's 0.733 -> 0.716 ms). At D = 128 the round trip saves two of the seven products but needs its two
+// kernels in sequence: it loses while the grid's longest chains, not its products, set the time,
+// which is the case up to two blocks of 128 rows per CU (1 x 8 x 1024: 39.9 against 58.8 us; 1 x 8 x
+// 8192, 512 blocks: 466 against 528; 640 blocks of T = 2048: 190 against 184; 1024: 489 against 428).
+inline bool workspace_recomputes(int T, int D, int pairs);
 hipError_t launch_backward_short(const BwdArgs& a, bool accumulate, hipStream_t s);
 
 // Dispatch chunk sizes, in workgroups per XCD group. The backward's is one round of resident
@@ -116,6 +125,11 @@ __host__ __device__ inline void decode_workgroup(int bid, int npairs, int nblk, 
 // free: ids that differ by a multiple of kCus start on the same CU.
 constexpr int kCus = 256;
 
+__host__ __device__ inline bool backward_is_short(int T, int D, int pairs) {
+  const int rounds = (pairs + kCus - 1) / kCus;
+  return D == 64 && T == 256 && pairs * 20 >= 19 * kCus * rounds;
+}
+
 // Item k of workgroup `bid` of a persistent grid of `grid` workgroups over npairs x nblk
 // (pair, block) items; false when the workgroup has fewer than k + 1 items. When both the pair
 // count and the grid are multiples of 8, the workgroups on XCD x (bid % 8 == x) serve the pairs
@@ -148,6 +162,20 @@ __host__ __device__ inline bool fwd_item_of(int bid, int grid, int k, int npairs
   return true;
 }
 
+// Index in the dQ grid of workgroup `bid` >= n1 of a grid of `grid` workgroups whose first n1 own
+// key blocks (bwd_both_kernel). Both grids go longest first. When all workgroups start at once (at
+// most `slots` per CU), the dQ blocks of every second row of kCus ids go shortest first instead, so
+// that a CU which starts a long block gets a short one beside it; eight ids at a time where the
+// grids are dealt by XCD (decode_workgroup), so that an id keeps its XCD.
+__host__ __device__ inline int both_dq_index(int bid, int n1, int grid, int slots) {
+  const int row = bid / kCus, i = bid - n1;
+  if ((row & 1) == 0 || grid > slots * kCus) return i;
+  const int lo = (row * kCus > n1 ? row * kCus : n1) - n1;
+  const int hi = ((row + 1) * kCus < grid ? (row + 1) * kCus : grid) - n1;
+  if (((n1 | grid) & 7) != 0) return lo + (hi - 1 - i);
+  return lo + (hi - 8 - (i & ~7)) + (i & 7);
+}
+
 constexpr int kFwdBlockM = 128;  // query rows per forward workgroup
 // The forward runs persistent (each resident workgroup takes items in turn, the next item's first
 // tiles loaded during the current item's last step) when there are at most this many (pair, query
@@ -157,6 +185,11 @@ constexpr int kFwdBlockM = 128;  // query rows per forward workgroup
 // 0.110 against 0.1155 ms) and at sixteen (T = 4096, D = 128).
 constexpr int kFwdPersistItems = 2;
 constexpr int kBwdBlockN = 128;  // keys owned by one dK/dV workgroup
+
+inline bool workspace_recomputes(int T, int D, int pairs) {
+  return D == 64 || (int64_t)pairs * ((T + kBwdBlockN - 1) / kBwdBlockN) <= 2 * kCus;
+}
+
 constexpr int kDqBlockM = 128;   // query rows owned by one dQ workgroup
 constexpr int kTile = 64;        // the reference's TILE_M = TILE_N (attention.metal:14-15)
 

@@ -49,11 +49,10 @@ extern "C" int flashAttentionBackwardNoAlloc(const uint16_t* dZ, const float* d,
   uint64_t need = 0;
   const int rc = metalllmAttnBackwardWorkspaceSize(p, &need);  // validates the shape
   if (rc) return rc;
-  // At D = 64 the workspace entry point never reads the workspace (M <= 256: the fused
-  // short-sequence backward keeps dS in LDS; longer: the recomputing kernels): any shape fits
+  // At D = 64 the workspace entry point never reads the workspace: any shape fits
   // there, and the nominal size is passed on so that the entry point's own size check accepts it
-  const int M = (int)p->M, D = (int)p->D;
-  const bool no_tiles = mla::backward_is_short(M, D) || mla::workspace_recomputes(M, D);
+  const int D = (int)p->D;
+  const bool no_tiles = D == 64;
   if (!no_tiles && need > kScratchBytes) return METALLLM_ATTN_E_SIZE;
   if (!dZ || !d || !l || !q || !k || !v || !dQ || !dK || !dV) return METALLLM_ATTN_E_NULL;
   if (!aligned16(dZ) || !aligned16(d) || !aligned16(l) || !aligned16(q) || !aligned16(k) || !aligned16(v) ||

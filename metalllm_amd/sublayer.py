@@ -14,8 +14,8 @@ from __future__ import annotations
 
 import ctypes
 
-from .attention import (AttentionParams, _check, _lib, _ptr, _stream, backward_part, computeD, flashAttentionForward,
-                        workspace_bytes)
+from .attention import (AttentionParams, _check, _lib, _ptr, _stream, computeD, flashAttentionBackwardWorkspace,
+                        flashAttentionForward, workspace_bytes)
 from .glue import castFloatToBfloat  # noqa: F401  (the dX handoff, model.h:692)
 
 _BOUND = False
@@ -240,11 +240,8 @@ class Sublayer:
         projBackwarddX(dOut, self.Wp, self.dO, p, stream)
         mark("proj")
         computeD(self.dO, self.o, self.Dv, stream, p)
-        # flashAttentionBackwardWorkspace, as its two kernels (the bench times them separately)
-        backward_part(2, self.dO, self.Dv, self.lse, self.q, self.k, self.v, self.dQ, self.dK, self.dV, stream, p,
-                      workspace=self.ws)
-        backward_part(3, self.dO, self.Dv, self.lse, self.q, self.k, self.v, self.dQ, self.dK, self.dV, stream, p,
-                      workspace=self.ws)
+        flashAttentionBackwardWorkspace(self.dO, self.Dv, self.lse, self.q, self.k, self.v, self.dQ, self.dK, self.dV,
+                                        self.ws, stream, p)
         mark("attention")
         computeGradDx(self.dX, self.Wq, self.Wk, self.Wv, self.dQ, self.dK, self.dV, p, stream)
         computeGradDw(self.X, self.dQ, self.dK, self.dV, self.dWq, self.dWk, self.dWv, p, stream)
