@@ -142,9 +142,9 @@ int flashAttentionBackwardNoAlloc(const uint16_t* dZ, const float* d, const floa
  * q, k, v, dK, dV, dAttn, out are bf16 [B*M, N]; dQ and dX are fp32 [B*M, N]; weights (q_w, k_w,
  * v_w, proj_w and their gradients) are bf16 [N, N] indexed [input feature][output feature], dQw
  * fp32 [N, N]. Products are computed with fp32 accumulation and rounded once to the destination
- * type: computeQKV, projForward and projBackwarddX on rocBLAS gemm_ex; computeGradDx,
- * computeGradDw and projBackwarddW on hand-written kernels when B*M and N are multiples of 128
- * (rocBLAS otherwise). The "accumulate" kernels read their destination once and add to it, as
+ * type: on hand-written kernels while N is a multiple of 64 and the product is small or fits no
+ * 128-wide tile; larger ones run computeGradDx, computeGradDw and projBackwarddW on hand-written
+ * kernels when B*M and N are multiples of 128, and the rest on rocBLAS gemm_ex. The "accumulate" kernels read their destination once and add to it, as
  * the reference's multiply_accumulate matmuls do; the caller zeroes those destinations first
  * (model.h:549-555). Validation: M, B, NH, D >= 1, N == NH*D a multiple of 8, tensors below 2^31
  * elements, non-NULL 16-byte aligned pointers. The first call on a device creates that device's
@@ -166,7 +166,8 @@ int metalllmSublayerReserve(const AttentionParams* p);
 /* attention.metal:19-53, dispatched at model.h:446-457: q = X.q_w, k = X.k_w, v = X.v_w. When
  * q_w, k_w, v_w are equally spaced in memory (e.g. slices of one [3][N][N] weight) and q, k, v
  * are equally spaced without overlapping (e.g. slices of one [3][B*M][N] buffer), the three
- * products run as one batched library call, which is faster; any other layout runs three. */
+ * products of a large call run as one batched library call, which is faster; any other layout runs
+ * three. Smaller calls run one hand-written launch on any layout. */
 int computeQKV(const uint16_t* X, uint16_t* q, uint16_t* k, uint16_t* v, const uint16_t* q_w, const uint16_t* k_w,
                const uint16_t* v_w, const AttentionParams* p, metalllm_stream_t stream);
 

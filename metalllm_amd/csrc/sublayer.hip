@@ -10,24 +10,28 @@
 // Row-major matrices: X, O, dZ, Q, K, V, dK, dV bf16 [R, C] and dQ, dX fp32 [R, C] with R = B*M rows
 // and C = N = NH*D features; weights bf16 [C, C] indexed [input feature][output feature].
 //
-// The bf16 GEMMs run on the platform library: rocBLAS gemm_ex with bf16 operands, fp32
-// accumulation and a bf16 or fp32 destination (beta = 1 for the reference's multiply_accumulate
-// kernels: the destination is read once and the sum rounded once). computeGradDx and computeGradDw
-// read the fp32 dQ, which the library cannot take as is: for row and feature counts that are
-// multiples of 128 they run hand-written matrix-core kernels (sublayer_gemm.hip) that load dQ as
-// fp32 and split it in registers into two bf16 terms, dQ = hi + lo + O(2^-16 |dQ|), each product
-// running on both; for other shapes a HIP kernel writes the same split to memory (split_dq) and
-// the library runs each product twice. Either way the fp32 dQ never makes a bf16 round trip.
+// Small products, and those whose row or feature counts fit no 128-wide tile, run hand-written kernels
+// on 64 x 64 tiles (sublayer_tile.hip; the rules below say which). The other bf16 GEMMs run on the
+// platform library: rocBLAS gemm_ex with bf16 operands, fp32 accumulation and a bf16 or fp32
+// destination (beta = 1 for the reference's multiply_accumulate kernels: the destination is read once
+// and the sum rounded once). computeGradDx and computeGradDw read the fp32 dQ, which the library
+// cannot take as is: larger ones whose row and feature counts are multiples of 128 run hand-written
+// kernels on 128-wide tiles (sublayer_gemm.hip). Both kinds split dQ in registers into two bf16
+// terms, dQ = hi + lo + O(2^-16 |dQ|), each product running on both; what is left (feature counts that
+// are no multiple of 64) writes the same split to memory (split_dq) and the library runs each product
+// twice. Either way the fp32 dQ never makes a bf16 round trip.
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 
 #include <algorithm>
+#include <cstdlib>
 #include <initializer_list>
 #include <mutex>
 #include <utility>
 #include <vector>
 
 #include "../../include/metalllm_attn.h"
+#include "sublayer_tile.hpp"
 
 namespace mla {  // attn_fwd.hip
 void forward_prepare();
@@ -202,6 +206,46 @@ int split_dq(const Ctx& c, const float* dQ, size_t elems, uint16_t* split) {
   return hipGetLastError() == hipSuccess ? METALLLM_ATTN_OK : METALLLM_ATTN_E_LAUNCH;
 }
 
+// Whether the 64 x 64 tile kernels (sublayer_tile.hip) take a product: up to large sizes where the
+// 128-wide kernels (sublayer_gemm.hip) and the library's large tiles do not fit, else small ones, which
+// they run in fewer and shorter dependent steps. A library call also costs about 21 us of host time,
+// these launches about 3. Device times, tile kernel against library or 128-wide kernel:
+//   rows, by units of 64 x 64 x 64: C = 768 computeQKV R = 1024 13 / 12 us, 2048 (13824 units) 19 / 17,
+//     4096 32 / 26; projForward 4096 12.0 / 14.6, 6144 (13824) 17 / 14; C = 384 computeQKV 8192 (13824)
+//     22 / 22, projForward 16384 (9216) 15.7 / 14.1; C = 448 computeQKV 8192 27 / 36, 16384 48 / 62
+//   computeGradDx, the dX + dW launch: C = 768 R = 2048 22 / 51, 6144 52 / 54, 8192 64 / 57 (with the
+//     weights break-even at 3072); C = 384 12288 32 / 32, 16384 38 / 35; C = 448 16384 49 / 92
+//   computeGradDw: C = 768 R = 2048 27 / 32, 4096 44 / 41; C = 384 16384 41 / 51; C = 448 16384 55 / 111
+//   projBackwarddW: C = 768 R = 4096 21 / 24, 8192 28 / 28, 16384 41 / 38; C = 384 16384 21 / 24
+bool tile_rows_ok(int R, int C, int n) {
+  return C % 64 == 0 && (int64_t)((R + 63) / 64) * (C / 64) * (C / 64) * n <= (C % 128 ? 64000 : 14000);
+}
+bool small_product(int R, int C, double limit) { return (double)R * C * C <= limit; }
+constexpr double kTileBeforeLibrary = 3e10;
+bool tile_dx_ok(int R, int C) {
+  return C % 64 == 0 && small_product(R, C, mla::grad_dx_fused_ok(R, C) ? 1.8e9 : kTileBeforeLibrary);
+}
+bool tile_dw_ok(int R, int C) {  // computeGradDw
+  const double limit = mla::grad_dw_fused_ok(R, C) ? (C <= 384 ? 3.6e9 : 1.8e9) : kTileBeforeLibrary;
+  return C % 64 == 0 && R % 64 == 0 && small_product(R, C, limit);
+}
+bool tile_dw_one_ok(int R, int C) {  // projBackwarddW
+  return C % 64 == 0 && R % 64 == 0 && small_product(R, C, mla::grad_dw_fused_ok(R, C) ? 4.8e9 : kTileBeforeLibrary);
+}
+// the phase encoder's launch of computeGradDx and the four weight gradients: where the entry point
+// takes them for dX, whose sums are then the same
+bool tile_dxdw_ok(int R, int C) { return R % 64 == 0 && tile_dx_ok(R, C); }
+
+int tile_rows(const Ctx& c, const mla::TileRows& a, bool wt) {
+  if (c.query) return METALLLM_ATTN_OK;
+  return mla::launch_tile_rows(a, wt, c.stream) == hipSuccess ? METALLLM_ATTN_OK : METALLLM_ATTN_E_LAUNCH;
+}
+
+int tile_grad(const Ctx& c, const mla::TileGrad& a, float* partial, bool accumulate) {
+  if (c.query) return METALLLM_ATTN_OK;
+  return mla::launch_tile_grad(a, partial, accumulate, c.stream) == hipSuccess ? METALLLM_ATTN_OK : METALLLM_ATTN_E_LAUNCH;
+}
+
 // Weight gradients W[k][n] += sum_r X[r][k] G[r][n] reduce over all R rows into a small C x C
 // output: one GEMM gives the library too few output tiles for the chip. The rows are split into
 // `parts` chunks, computed as one strided-batched GEMM into fp32 partials [chunk][C][C], and
@@ -213,17 +257,24 @@ int row_chunks(int R) {
   return 1;
 }
 
-// Elements of the dQ split (hi, then lo) that the library paths of computeGradDx and
-// computeGradDw read: none when the hand-written kernels take the shape (they split in registers).
-size_t split_need(int R, int C) {
-  return mla::grad_dx_fused_ok(R, C) && mla::grad_dw_fused_ok(R, C) ? 0 : 2 * (size_t)R * C;
+// Elements of the dQ split (hi, then lo) that the library paths of computeGradDx (dx) and
+// computeGradDw read: none where the hand-written kernels take the shape (they split in registers).
+size_t split_need(int R, int C, bool dx) {
+  const bool ok = dx ? tile_dx_ok(R, C) || mla::grad_dx_fused_ok(R, C) : tile_dw_ok(R, C) || mla::grad_dw_fused_ok(R, C);
+  return ok ? 0 : 2 * (size_t)R * C;
 }
 
-// fp32 partial floats for projBackwarddW and computeGradDw: the hand-written kernel's chunks, or
-// row_chunks(R) products of C x C (twice that for computeGradDw's dQw) on the library path.
+// fp32 partial floats for projBackwarddW, computeGradDw and the encoder's launch: the hand-written
+// kernels' chunks, or row_chunks(R) products of C x C (twice that for computeGradDw's dQw) on the
+// library path.
 size_t partial_need(int R, int C) {
+  const size_t tile = C % 64 || R % 64 ? 0
+                                       : std::max({mla::tile_grad_partial_floats(R, C, 3, 4, false),
+                                                   mla::tile_grad_partial_floats(R, C, 0, 3, false),
+                                                   mla::tile_grad_partial_floats(R, C, 0, 4, true)});
+  if (tile_dw_one_ok(R, C) && tile_dw_ok(R, C) && tile_dxdw_ok(R, C)) return tile;
   if (mla::grad_dw_fused_ok(R, C))
-    return std::max({mla::grad_dw_one_partial_floats(R, C), mla::grad_dw_partial_floats(R, C),
+    return std::max({tile, mla::grad_dw_one_partial_floats(R, C), mla::grad_dw_partial_floats(R, C),
                      mla::grad_dw4_partial_floats(R, C)});
   return 2 * (size_t)row_chunks(R) * C * C;
 }
@@ -292,6 +343,9 @@ int op_qkv(const Ctx& c, const uint16_t* X, uint16_t* q, uint16_t* k, uint16_t* 
            const uint16_t* k_w, const uint16_t* v_w, int R, int C) {
   // distances in bf16 elements, from the integer addresses (the buffers may be separate allocations)
   const auto at = [](const uint16_t* ptr) { return (intptr_t)(uintptr_t)ptr; };
+  const auto apart = [&](const uint16_t* a, const uint16_t* b) { return std::abs(at(a) - at(b)) >= 2 * (intptr_t)R * C; };
+  if (tile_rows_ok(R, C, 3) && apart(q, k) && apart(k, v) && apart(q, v))
+    return tile_rows(c, mla::TileRows{X, {q_w, k_w, v_w}, {q, k, v}, 3, R, C}, false);
   const intptr_t bw = at(k_w) - at(q_w), by = at(k) - at(q);
   const intptr_t dw = bw / 2, dy = by / 2;
   if (bw % 2 == 0 && by % 2 == 0 && dw >= 0 && at(v_w) - at(k_w) == bw && dy >= (intptr_t)R * C &&
@@ -310,15 +364,20 @@ int op_qkv(const Ctx& c, const uint16_t* X, uint16_t* q, uint16_t* k, uint16_t* 
 }
 
 int op_proj_fwd(const Ctx& c, const uint16_t* attn_out, const uint16_t* proj_w, uint16_t* out, int R, int C) {
+  if (tile_rows_ok(R, C, 1)) return tile_rows(c, mla::TileRows{attn_out, {proj_w}, {out}, 1, R, C}, false);
   return gemm_rm(c, false, false, R, C, C, attn_out, BF, C, proj_w, BF, C, 0.0f, out, BF, C);
 }
 
 // partial: at least partial_need(R, C) floats. accumulate = false: dProjw is written as if it
-// held zeros (the phase encoder; every op_* below takes the same flag). Row counts that are
-// multiples of 128 and feature counts that are multiples of 128 run computeGradDw's hand-written
-// kernel (sublayer_gemm.hip) on the one bf16 gradient; other shapes use the library.
+// held zeros (the phase encoder; every op_* below takes the same flag). Larger products in multiples
+// of 128 run computeGradDw's 128-wide kernel (sublayer_gemm.hip) on the one bf16 gradient.
 int op_proj_dw(const Ctx& c, const uint16_t* attn_out, const uint16_t* dZ, uint16_t* dProjw, int R, int C,
                float* partial, bool accumulate = true) {
+  if (tile_dw_one_ok(R, C)) {
+    mla::TileGrad a{};
+    a.x[3] = attn_out, a.g[3] = dZ, a.dW[3] = dProjw, a.w0 = 3, a.w1 = 4, a.R = R, a.C = C;
+    return tile_grad(c, a, partial, accumulate);
+  }
   if (mla::grad_dw_fused_ok(R, C)) {
     if (c.query) return METALLLM_ATTN_OK;
     return mla::launch_grad_dw_one(attn_out, dZ, dProjw, partial, R, C, accumulate, c.stream) == hipSuccess
@@ -331,15 +390,17 @@ int op_proj_dw(const Ctx& c, const uint16_t* attn_out, const uint16_t* dZ, uint1
 }
 
 int op_proj_dx(const Ctx& c, const uint16_t* dZ, const uint16_t* proj_w, uint16_t* dAttn, int R, int C) {
+  if (tile_rows_ok(R, C, 1)) return tile_rows(c, mla::TileRows{dZ, {proj_w}, {dAttn}, 1, R, C}, true);
   return gemm_rm(c, false, true, R, C, C, dZ, BF, C, proj_w, BF, C, 0.0f, dAttn, BF, C);
 }
 
-// Row and feature counts that are multiples of 128 run the hand-written kernel (sublayer_gemm.hip),
-// which reads the fp32 dQ itself; other shapes use the library on hi, lo, the two-term bf16 split
-// of dQ (split_dq).
+// The hand-written kernels read the fp32 dQ themselves; the library runs on hi, lo, the two-term bf16
+// split of dQ (split_dq).
 int op_grad_dx(const Ctx& c, float* dX, const uint16_t* qw, const uint16_t* kw, const uint16_t* vw, const float* dQ,
                const uint16_t* hi, const uint16_t* lo, const uint16_t* dK, const uint16_t* dV, int R, int C,
                bool accumulate = true) {
+  if (tile_dx_ok(R, C))
+    return tile_grad(c, mla::TileGrad{dX, dQ, {qw, kw, vw}, {}, {nullptr, dK, dV}, {}, 0, 0, R, C}, nullptr, accumulate);
   if (mla::grad_dx_fused_ok(R, C)) {
     if (c.query) return METALLLM_ATTN_OK;
     return mla::launch_grad_dx(dX, dQ, dK, dV, qw, kw, vw, R, C, accumulate, c.stream) == hipSuccess
@@ -352,12 +413,13 @@ int op_grad_dx(const Ctx& c, float* dX, const uint16_t* qw, const uint16_t* kw, 
   return gemm_rm(c, false, true, R, C, C, dV, BF, C, vw, BF, C, 1.0f, dX, F32, C);
 }
 
-// partial: at least partial_need(R, C) floats. Row counts that are multiples of 128 and feature
-// counts that are multiples of 128 run the hand-written kernel (sublayer_gemm.hip) on the fp32 dQ;
-// other shapes use the library on hi, lo, the two-term bf16 split of dQ (split_dq).
+// partial: at least partial_need(R, C) floats; hi, lo as in op_grad_dx.
 int op_grad_dw(const Ctx& c, const uint16_t* x, const float* dQ, const uint16_t* hi, const uint16_t* lo,
                const uint16_t* dK, const uint16_t* dV, float* dQw, uint16_t* dKw, uint16_t* dVw, int R, int C,
                float* part, bool accumulate = true) {
+  if (tile_dw_ok(R, C))
+    return tile_grad(c, mla::TileGrad{nullptr, dQ, {}, {x, x, x}, {nullptr, dK, dV}, {dQw, dKw, dVw}, 0, 3, R, C}, part,
+                     accumulate);
   if (mla::grad_dw_fused_ok(R, C)) {
     if (c.query) return METALLLM_ATTN_OK;
     return mla::launch_grad_dw(x, dQ, dK, dV, dQw, dKw, dVw, part, R, C, accumulate, c.stream) == hipSuccess
@@ -467,7 +529,7 @@ int computeGradDx(float* dX, const uint16_t* qw, const uint16_t* kw, const uint1
   const size_t e = (size_t)R * C;
   Public u(stream);
   TRY(u.s.rc);
-  if (mla::grad_dx_fused_ok(R, C)) return op_grad_dx(u.c, dX, qw, kw, vw, dQ, nullptr, nullptr, dK, dV, R, C);
+  if (!split_need(R, C, true)) return op_grad_dx(u.c, dX, qw, kw, vw, dQ, nullptr, nullptr, dK, dV, R, C);
   TRY(ensure(u.s.st->split, u.s.st->split_elems, 2 * e, u.c.stream));
   TRY(split_dq(u.c, dQ, e, u.s.st->split));
   return op_grad_dx(u.c, dX, qw, kw, vw, dQ, u.s.st->split, u.s.st->split + e, dK, dV, R, C);
@@ -482,7 +544,7 @@ int computeGradDw(const uint16_t* x, const float* dQ, const uint16_t* dK, const 
   Public u(stream);
   TRY(u.s.rc);
   TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial_need(R, C), u.c.stream));
-  if (mla::grad_dw_fused_ok(R, C))
+  if (!split_need(R, C, false))
     return op_grad_dw(u.c, x, dQ, nullptr, nullptr, dK, dV, dQw, dKw, dVw, R, C, u.s.st->partial);
   TRY(ensure(u.s.st->split, u.s.st->split_elems, 2 * e, u.c.stream));
   TRY(split_dq(u.c, dQ, e, u.s.st->split));
@@ -564,7 +626,8 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
   // balanced items instead of projBackwarddW's own short-item launch. Its sum then runs over
   // other row chunks than the entry point's, so it can differ from projBackwarddW's result by the
   // fp32 summation order (one bf16 rounding step at most).
-  const bool fuse_pdw = mla::grad_dw_fused_ok(R, C) && mla::grad_dx_fused_ok(R, C);
+  const bool tile = tile_dxdw_ok(R, C);
+  const bool fuse_pdw = tile || (mla::grad_dw_fused_ok(R, C) && mla::grad_dx_fused_ok(R, C));
   if (!fuse_pdw) TRY(op_proj_dw(c, b->attn_out, b->dOut, b->dProjw, R, C, partial, false));
   TRY(op_proj_dx(c, b->dOut, b->proj_w, b->dAttn, R, C));
   if (!c.query) {
@@ -573,13 +636,16 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
                                         attn_ws_bytes, p, s));
   }
   uint16_t* lo = nullptr;  // no split when both hand-written kernels take the shape
-  if (split_need(R, C)) {
+  if (!tile && std::max(split_need(R, C, true), split_need(R, C, false))) {
     TRY(split_dq(c, b->dQ, e, split));  // one split serves both consumers
     lo = split + e;
   } else {
     split = nullptr;
   }
-  if (fuse_pdw) {
+  if (tile) {
+    TRY(tile_grad(c, mla::TileGrad{b->dX, b->dQ, {b->q_w, b->k_w, b->v_w}, {b->X, b->X, b->X, b->attn_out},
+                                   {nullptr, b->dK, b->dV, b->dOut}, {b->dQw, b->dKw, b->dVw, b->dProjw}, 0, 4, R, C}, partial, false));
+  } else if (fuse_pdw) {
     // computeGradDx and the four weight gradients in one launch (dX tiles first, then the
     // weight-gradient items, which start as the dX tiles finish), then the reduction
     if (!c.query && mla::launch_grad_dxdw4(b->dX, b->X, b->dQ, b->dK, b->dV, b->q_w, b->k_w, b->v_w, b->attn_out,
@@ -607,12 +673,13 @@ int build_graph(metalllmSublayerGraph* g, const metalllmSublayerBuffers* b, cons
     return METALLLM_ATTN_E_LIBRARY;
   }
   if (g->phase == 1) {
-    const size_t split = split_need(R, C);
+    const size_t split = std::max(split_need(R, C, true), split_need(R, C, false));
     if (split && hipMalloc((void**)&g->split, split * sizeof(uint16_t)) != hipSuccess) g->split = nullptr;
-    if (hipMalloc((void**)&g->partial, partial_need(R, C) * sizeof(float)) != hipSuccess) g->partial = nullptr;
+    const size_t partial = partial_need(R, C);
+    if (partial && hipMalloc((void**)&g->partial, partial * sizeof(float)) != hipSuccess) g->partial = nullptr;
     TRY(metalllmAttnBackwardWorkspaceSize(p, &g->attn_ws_bytes));
     if (hipMalloc(&g->attn_ws, g->attn_ws_bytes) != hipSuccess) g->attn_ws = nullptr;
-    if ((split && !g->split) || !g->partial || !g->attn_ws) return METALLLM_ATTN_E_LIBRARY;
+    if ((split && !g->split) || (partial && !g->partial) || !g->attn_ws) return METALLLM_ATTN_E_LIBRARY;
   }
   // the workspace the phase's rocBLAS calls need, owned by the graph
   size_t ws = 0;
@@ -657,7 +724,7 @@ int metalllmSublayerEncode(int phase, const metalllmSublayerBuffers* b, const At
   TRY(u.s.rc);
   uint64_t ws = 0;
   if (phase == 1) {
-    TRY(ensure(u.s.st->split, u.s.st->split_elems, split_need(R, C), u.c.stream));
+    TRY(ensure(u.s.st->split, u.s.st->split_elems, std::max(split_need(R, C, true), split_need(R, C, false)), u.c.stream));
     TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial_need(R, C), u.c.stream));
     TRY(metalllmAttnBackwardWorkspaceSize(p, &ws));
     TRY(ensure(u.s.st->attn_ws, u.s.st->attn_ws_bytes, (size_t)ws, u.c.stream));
@@ -674,8 +741,11 @@ int metalllmSublayerReserve(const AttentionParams* p) {
   TRY(metalllmAttnBackwardWorkspaceSize(p, &ws));
   Public u(nullptr);
   TRY(u.s.rc);
-  TRY(ensure(u.s.st->split, u.s.st->split_elems, split_need(R, C), nullptr));
-  TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial_need(R, C), nullptr));
+  // what the library path of this shape would take too: a smaller shape may run it
+  const bool lib = !mla::grad_dw_fused_ok(R, C);
+  const size_t partial = std::max(partial_need(R, C), lib ? 2 * (size_t)row_chunks(R) * C * C : 0);
+  TRY(ensure(u.s.st->split, u.s.st->split_elems, lib ? 2 * (size_t)R * C : 0, nullptr));
+  TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial, nullptr));
   TRY(ensure(u.s.st->attn_ws, u.s.st->attn_ws_bytes, (size_t)ws, nullptr));
   return METALLLM_ATTN_OK;
 }

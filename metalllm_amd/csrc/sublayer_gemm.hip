@@ -563,6 +563,15 @@ int device_cus() {
 
 }  // namespace
 
+// Adds the partials [nq + others * nkv][C][C] of the weights w0 .. w0 + nw - 1 (grad_dw_reduce_kernel).
+hipError_t launch_grad_dw_reduce(const float* part, float* dQw, uint16_t* dKw, uint16_t* dVw, uint16_t* dPw, int C, int nq,
+                                 int nkv, int w0, int nw, bool accumulate, hipStream_t s) {
+  const size_t cc = (size_t)C * C, n4 = nw * cc / 4;
+  hipLaunchKernelGGL(grad_dw_reduce_kernel, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096)), dim3(256), 0, s, part,
+                     dQw, dKw, dVw, dPw, C, nq, nkv, w0, nw, accumulate);
+  return hipGetLastError();
+}
+
 bool grad_dx_fused_ok(int R, int C) { return R % kGxTile == 0 && C % kGxTile == 0; }
 
 bool grad_dw_fused_ok(int R, int C) { return R % (2 * kGwK) == 0 && C % kGwTile == 0; }
