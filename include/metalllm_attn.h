@@ -112,7 +112,7 @@ int metalllmAttnBackwardWorkspaceSize(const AttentionParams* p, uint64_t* bytes)
  * holds no state between calls, but one
  * workspace must not serve two calls at once. Returns METALLLM_ATTN_E_NULL / _E_ALIGN / _E_SIZE
  * for a NULL, misaligned or too small workspace. At D = 64, and at D = 128 while B*NH*ceil(M/128) is
- * at most 512 (two workgroups per CU), no dS is stored and the workspace is validated but not used:
+ * at most 512 (384 for M < 512), no dS is stored and the workspace is validated but not used:
  * it runs flashAttentionBackward's kernel writing dQ instead of adding into it (there the
  * recomputation in one launch is faster than the dS round trip's two), so dQ, dK and dV equal
  * flashAttentionBackward's into a zeroed dQ bit for bit.

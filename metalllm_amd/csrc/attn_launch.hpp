@@ -71,7 +71,9 @@ __host__ __device__ inline bool backward_is_short(int T, int D, int pairs);
 // 4's 0.733 -> 0.716 ms). At D = 128 the round trip saves two of the seven products but needs its two
 // kernels in sequence: it loses while the grid's longest chains, not its products, set the time,
 // which is the case up to two blocks of 128 rows per CU (1 x 8 x 1024: 39.9 against 58.8 us; 1 x 8 x
-// 8192, 512 blocks: 466 against 528; 640 blocks of T = 2048: 190 against 184; 1024: 489 against 428).
+// 8192, 512 blocks: 466 against 528; 640 blocks of T = 2048: 190 against 184; 1024: 489 against 428),
+// and up to one and a half where T < 512 (384 blocks of T = 128, 256, 384: 34.4, 38.3, 41.2 against
+// 33.6, 38.5, 44.4 us; 512 blocks: 43.2, 53.1, 55.3 against 38.8, 45.3, 52.6).
 inline bool workspace_recomputes(int T, int D, int pairs);
 hipError_t launch_backward_short(const BwdArgs& a, bool accumulate, hipStream_t s);
 
@@ -187,7 +189,7 @@ constexpr int kFwdPersistItems = 2;
 constexpr int kBwdBlockN = 128;  // keys owned by one dK/dV workgroup
 
 inline bool workspace_recomputes(int T, int D, int pairs) {
-  return D == 64 || (int64_t)pairs * ((T + kBwdBlockN - 1) / kBwdBlockN) <= 2 * kCus;
+  return D == 64 || (int64_t)pairs * ((T + kBwdBlockN - 1) / kBwdBlockN) <= (T >= 512 ? 2 * kCus : kCus * 3 / 2);
 }
 
 constexpr int kDqBlockM = 128;   // query rows owned by one dQ workgroup

@@ -18,6 +18,8 @@ pytestmark = pytest.mark.gpu
     (7, 192, 23, 64, 1),     # 322 + 322, last row partial
     (3, 960, 11, 128, 1),    # 264 + 264: more than two per CU, in list order
     (65, 448, 2, 128, 1),    # 520 blocks: dS stored, two-tile dQ ring
+    (23, 256, 8, 128, 1),    # 368 blocks: below the line of T < 512 (384)
+    (25, 256, 8, 128, 1),    # 400 blocks: above it
     (9, 576, 13, 128, 1),    # 585 blocks: dS stored, four-tile ring, last item 1 of 4 tiles
     (122, 256, 2, 64, 1),    # 244 pairs: the fused T = 256 kernel, one round 95% full
     (121, 256, 2, 64, 1),    # 242 pairs: below that line
