@@ -95,14 +95,16 @@ def _ptr(t):
         raise ValueError("tensor must live on the GPU")
     if not t.is_contiguous():
         raise ValueError("tensor must be contiguous")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _stream(stream):
-    import torch
+    """The stream's handle; None: the current device's current stream, by its raw handle (building
+    the torch.cuda.Stream object took 3 us of an 8.4 us call)."""
     if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+        import torch
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    return stream.cuda_stream
 
 
 def _shape(q):

@@ -196,7 +196,7 @@ class Sublayer:
         for n in blk:
             t[n] = getattr(self, n) if self.hidden is not None else None
         for n in SublayerBuffers.FIELDS:
-            setattr(b, n, _ptr(t[n]).value if t[n] is not None else None)
+            setattr(b, n, _ptr(t[n]))
         b.ln_eps = self.ln_eps
         return b
 
