@@ -494,10 +494,11 @@ hipError_t launch_forward(const FwdArgs& a, int D, hipStream_t s) {
   const int res = D == 64 ? fwd_resident<64>() : fwd_resident<128>();
   if (res <= 0) return hipErrorInvalidDevice;
   if (items <= kFwdPersistItems * res) {
-    // as many workgroups as are resident at once (a multiple of 8, so that pairs keep to one
-    // XCD), or one per item when there are fewer items
-    int grid = std::min(items, res);
-    if (grid >= 8) grid -= grid % 8;
+    // as many workgroups as are resident at once (a multiple of 8, so that pairs keep to one XCD), or
+    // one per item when there are fewer items: rounded down as well, 12 items ran on 8 workgroups, two
+    // in a row on four of them (B = 1, H = 6, T = 256: 10.4 us, 7.1 us with 12)
+    int grid = items;
+    if (items > res) grid = res >= 8 ? res - res % 8 : res;
     if (D == 64)
       hipLaunchKernelGGL((fwd_kernel<64, true>), dim3((unsigned)grid), dim3(256), 0, s, a);
     else
