@@ -32,6 +32,7 @@ __global__ void __launch_bounds__(256) compute_d_kernel(ComputeDArgs a, uint64_t
   const uint64_t gid = (uint64_t)blockIdx.x * 256u + threadIdx.x;
   const uint64_t row = gid >> 2;  // (b*T + t)*H + h: rows of [B,T,H,D] are contiguous
   const int j = (int)(gid & 3);
+  if (gid < a.n_zero) a.zero0[gid] = a.zero1[gid] = 0.0f;
   float acc[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.0f;

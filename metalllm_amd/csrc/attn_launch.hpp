@@ -22,6 +22,10 @@ struct ComputeDArgs {
   const uint16_t* O;
   float* Dv;
   int T, H, B;
+  // optional: n_zero floats each set to 0 by the same launch (the phase encoder's layernorm gradients)
+  float* zero0 = nullptr;
+  float* zero1 = nullptr;
+  uint32_t n_zero = 0;
 };
 
 struct BwdArgs {

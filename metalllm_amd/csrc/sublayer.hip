@@ -25,17 +25,12 @@
 
 #include <algorithm>
 #include <cstdlib>
-#include <initializer_list>
 #include <mutex>
-#include <utility>
 #include <vector>
 
 #include "../../include/metalllm_attn.h"
+#include "attn_launch.hpp"
 #include "sublayer_tile.hpp"
-
-namespace mla {  // attn_fwd.hip
-void forward_prepare();
-}  // namespace mla
 
 namespace mla {  // glue.hip
 hipError_t launch_block_ln_bwd(const float* dX, const uint16_t* dOut, const uint16_t* xnorm, const uint16_t* gamma,
@@ -438,37 +433,6 @@ int op_grad_dw(const Ctx& c, const uint16_t* x, const float* dQ, const uint16_t*
   return reduce_into(c, part, parts, cc, dVw, true, accumulate);
 }
 
-// Zeroes up to 8 buffers in one launch (a fill kernel: no memset node when captured into a
-// graph). Each segment is n16 16-byte words; grid-stride over each segment in turn.
-struct ZeroSet {
-  uint4* p[8];
-  size_t n16[8];
-  int n;
-};
-
-__global__ void __launch_bounds__(256) zero_kernel(ZeroSet z) {
-  const size_t stride = (size_t)gridDim.x * blockDim.x, i0 = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  for (int k = 0; k < z.n; ++k)
-    for (size_t i = i0; i < z.n16[k]; i += stride) z.p[k][i] = uint4{0u, 0u, 0u, 0u};
-}
-
-// (pointer, bytes) pairs, bytes a multiple of 16
-int zero_buffers(const Ctx& c, std::initializer_list<std::pair<void*, size_t>> bufs) {
-  if (c.query) return METALLLM_ATTN_OK;
-  ZeroSet z{};
-  size_t largest = 0;
-  for (const auto& b : bufs) {
-    if (z.n == 8) return METALLLM_ATTN_E_LAUNCH;
-    z.p[z.n] = (uint4*)b.first;
-    z.n16[z.n] = b.second / 16;
-    largest = std::max(largest, z.n16[z.n]);
-    ++z.n;
-  }
-  const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>((largest + 255) / 256, 8192));
-  hipLaunchKernelGGL(zero_kernel, dim3(blocks), dim3(256), 0, c.stream, z);
-  return hipGetLastError() == hipSuccess ? METALLLM_ATTN_OK : METALLLM_ATTN_E_LAUNCH;
-}
-
 // Public entry points: the device's handle and buffers, bound to the caller's stream.
 struct Public {
   Session s;
@@ -610,6 +574,12 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
       TRY(layernormForward(b->hidden, b->ln_xnorm, (uint16_t*)b->X, b->ln_gamma, b->ln_beta, b->ln_stdev, &lp, s));
     TRY(op_qkv(c, b->X, b->q, b->k, b->v, b->q_w, b->k_w, b->v_w, R, C));
     if (!c.query) TRY(flashAttentionForward(b->q, b->k, b->v, b->attn_out, b->l, p, s));
+    if (block && tile_rows_ok(R, C, 1)) {  // the projection's tiles add hidden as they are stored (model.h:483)
+      mla::TileRows t{b->attn_out, {b->proj_w}, {b->out}, 1, R, C};
+      t.add = b->hidden;
+      t.sum = b->residual;
+      return tile_rows(c, t, false);
+    }
     TRY(op_proj_fwd(c, b->attn_out, b->proj_w, b->out, R, C));
     if (block && !c.query) TRY(residualAdd(b->hidden, b->out, b->residual, (uint32_t)e, s));  // model.h:483
     return METALLLM_ATTN_OK;
@@ -619,8 +589,7 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
   // runs them in write mode instead: the result is bit for bit 0 + the gradient (-0 becomes +0),
   // without the zeroing pass and without reading the destinations. The attention backward writes
   // dQ, dK and dV in full; the block's layernorm gradients (model.h:545-546), which its backward
-  // adds into with atomics, are zeroed here.
-  if (block) TRY(zero_buffers(c, {{b->ln_dgamma, (size_t)C * 4}, {b->ln_dbeta, (size_t)C * 4}}));
+  // adds into with atomics, are zeroed by computeD's launch.
   // With the hand-written weight-gradient kernel, dProjw (which nothing in this phase reads) is
   // computed at the end, as a fourth weight of computeGradDw's launch and reduction: one launch of
   // balanced items instead of projBackwarddW's own short-item launch. Its sum then runs over
@@ -629,9 +598,25 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
   const bool tile = tile_dxdw_ok(R, C);
   const bool fuse_pdw = tile || (mla::grad_dw_fused_ok(R, C) && mla::grad_dx_fused_ok(R, C));
   if (!fuse_pdw) TRY(op_proj_dw(c, b->attn_out, b->dOut, b->dProjw, R, C, partial, false));
-  TRY(op_proj_dx(c, b->dOut, b->proj_w, b->dAttn, R, C));
+  // projBackwarddX and computeD: one launch where the tiles of dAttn are whole heads
+  float *dgamma = block ? b->ln_dgamma : nullptr, *dbeta = block ? b->ln_dbeta : nullptr;
+  if (tile_rows_ok(R, C, 1) && p->D == 64) {
+    mla::TileRows t{b->dOut, {b->proj_w}, {b->dAttn}, 1, R, C};
+    t.O = b->attn_out;
+    t.Dv = b->Dsum;
+    t.T = (int)p->M;
+    t.H = (int)p->NH;
+    t.zero0 = dgamma;
+    t.zero1 = dbeta;
+    TRY(tile_rows(c, t, true));
+  } else {
+    TRY(op_proj_dx(c, b->dOut, b->proj_w, b->dAttn, R, C));
+    if (!c.query && mla::launch_compute_d(mla::ComputeDArgs{b->dAttn, b->attn_out, b->Dsum, (int)p->M, (int)p->NH,
+                                                            (int)p->B, dgamma, dbeta, block ? (uint32_t)C : 0u},
+                                          (int)p->D, c.stream) != hipSuccess)
+      return METALLLM_ATTN_E_LAUNCH;
+  }
   if (!c.query) {
-    TRY(computeD(b->dAttn, b->attn_out, b->Dsum, p, s));
     TRY(flashAttentionBackwardWorkspace(b->dAttn, b->Dsum, b->l, b->q, b->k, b->v, b->dQ, b->dK, b->dV, attn_ws,
                                         attn_ws_bytes, p, s));
   }

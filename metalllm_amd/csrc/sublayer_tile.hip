@@ -128,6 +128,11 @@ __device__ __forceinline__ void wait_lds() {
   asm volatile("" ::: "memory");
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false));
+}
+
 // acc[tc][tp]: c 32tc + 8g + 4h + i (register 4g + i), p 32tp + l32
 struct Acc {
   f32x16 v[2][2];
@@ -224,10 +229,44 @@ __global__ void __launch_bounds__(64 * NW, 2) tile_rows_kernel(TileRows a) {
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) products(acc, A[ks], B[ks]);
   }
+  if (a.zero0 && item == 0)
+    for (int i = tid; i < a.C; i += 64 * NW) a.zero0[i] = a.zero1[i] = 0.0f;
   uint16_t* out = a.y[y];
   reduce_tiles<NW>(L, tid, wave, smem, acc, [&](int p, int c, f32x4 s) {
-    if (r0 + p < a.R)
-      *(u32x2*)(out + (size_t)(r0 + p) * a.C + c0 + c) = u32x2{pack_bf16(s[0], s[1]), pack_bf16(s[2], s[3])};
+    const bool live = r0 + p < a.R;
+    const size_t o = (size_t)(live ? r0 + p : a.R - 1) * a.C + c0 + c;  // past the end: read in bounds, not stored
+    const u32x2 v = {pack_bf16(s[0], s[1]), pack_bf16(s[2], s[3])};
+    if (live) *(u32x2*)(out + o) = v;
+    if (a.sum) {
+      const u32x2 x = *(const u32x2*)(a.add + o);
+      if (live)
+        *(u32x2*)(a.sum + o) = u32x2{pack_bf16(bf_lo(x[0]) + bf_lo(v[0]), bf_hi(x[0]) + bf_hi(v[0])),
+                                     pack_bf16(bf_lo(x[1]) + bf_lo(v[1]), bf_hi(x[1]) + bf_hi(v[1]))};
+    }
+    if (a.Dv) {
+      // computeD's sum (attn_computed.hip) bit for bit: columns l and l + 32 first, from 0, then the
+      // butterfly over the 32 sums. The 16 lanes of a row hold columns 4 k .. 4 k + 3 (k = lane % 16):
+      // l + 32 is lane k + 8, distances 16, 8, 4 are lanes k ^ 4, k ^ 2, k ^ 1, and 2, 1 in-lane. The
+      // rotations reach the partners because lanes k and k ^ 8 hold the same sums by then.
+      const u32x2 y = *(const u32x2*)(a.O + o);
+      const uint32_t p0 = pack_bf16(bf_lo(v[0]) * bf_lo(y[0]), bf_hi(v[0]) * bf_hi(y[0]));
+      const uint32_t p1 = pack_bf16(bf_lo(v[1]) * bf_lo(y[1]), bf_hi(v[1]) * bf_hi(y[1]));
+      float d[4] = {bf_lo(p0), bf_hi(p0), bf_lo(p1), bf_hi(p1)};
+      const float zero = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (c < 32) d[i] = zero + d[i];
+        d[i] += dpp_move<0x128>(d[i]);  // row_ror:8
+        d[i] += dpp_move<0x124>(d[i]);  // row_ror:4
+        d[i] += dpp_move<0x4e>(d[i]);   // quad_perm 2,3,0,1
+        d[i] += dpp_move<0xb1>(d[i]);   // quad_perm 1,0,3,2
+      }
+      const float total = (d[0] + d[2]) + (d[1] + d[3]);
+      if (live && c == 0) {
+        const int r = r0 + p, b = r / a.T;
+        a.Dv[((size_t)b * a.H + ct) * a.T + (r - b * a.T)] = bf_lo(pack_bf16(total, total));
+      }
+    }
   });
 }
 

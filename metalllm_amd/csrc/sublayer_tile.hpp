@@ -11,6 +11,13 @@ struct TileRows {
   const uint16_t* w[3];
   uint16_t* y[3];
   int n, R, C;
+  // the phase encoder's additions to a product of one weight, all optional:
+  const uint16_t* add;  // sum[r][n] = bf16(add + Y) (residualAdd)
+  uint16_t* sum;
+  const uint16_t* O;  // heads of 64 features: Dv[b][h][t] = computeD of Y and O, H heads, T rows a batch
+  float* Dv;
+  int T, H;
+  float *zero0, *zero1;  // C floats each set to 0
 };
 // wt: W_i indexed [n][k], else [k][n].
 hipError_t launch_tile_rows(const TileRows& a, bool wt, hipStream_t s);

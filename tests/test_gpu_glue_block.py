@@ -1,7 +1,7 @@
 """layernormBackward where a row is shared by one, two and four waves, with row counts that leave the
 last step of a workgroup partly empty, against the oracle at the bars of test_gpu_glue.py; and the
-phase encoder's form (dX cast, ln1 backward and skip add in one kernel) bit for bit against the
-three public calls on the encoder's own dX."""
+phase encoder's forms (dX cast, ln1 backward and skip add in one kernel; computeD and the residual
+add in the projections' launches) bit for bit against the public calls on the encoder's own tensors."""
 import numpy as np
 import pytest
 
@@ -18,8 +18,11 @@ def test_layernorm_row_split(gpu, rows, cols):
     glue_checks.test_layernorm_forward_backward(gpu, G, rows, cols, 1.0)
 
 
-@pytest.mark.parametrize("B,T,H,C", [(1, 64, 1, 64), (3, 192, 6, 384), (2, 64, 12, 768), (1, 128, 20, 1280), (1, 64, 20, 2560)])
-def test_block_backward_end(gpu, B, T, H, C):
+@pytest.mark.parametrize("B,T,H,C", [(1, 64, 1, 64), (3, 192, 6, 384), (2, 64, 12, 768), (1, 128, 20, 1280), (1, 64, 20, 2560),
+                                     (8, 1024, 12, 768), (3, 320, 5, 320), (2, 192, 3, 384)])
+def test_block_ends(gpu, B, T, H, C):
+    """Also computeD and the residual add where the projections' tiles do them (D = 64; residual at
+    every D), against the public calls on the encoder's own dAttn, attn_out and out."""
     import torch
     import metalllm_amd.glue as G
     import metalllm_amd.sublayer as S
@@ -35,7 +38,13 @@ def test_block_backward_end(gpu, B, T, H, C):
     G.castFloatToBfloat(blk.dX, d)
     G.layernormBackward(d, blk.ln_xnorm, blk.ln_gamma, blk.ln_stdev, dg, db)
     G.residualAdd(d, blk.dOut, d)
+    import metalllm_amd as M
+    Dv, res = torch.empty_like(blk.Dv), torch.empty_like(blk.residual)
+    four = lambda t: t.view(B, T, H, C // H)
+    M.computeD(four(blk.dO), four(blk.o), Dv)
+    G.residualAdd(blk.hidden, blk.out, res)
     torch.cuda.synchronize()
-    assert torch.equal(d, blk.dStream)
+    assert torch.equal(d, blk.dStream) and torch.equal(res, blk.residual)
+    assert torch.equal(Dv.view(torch.int32), blk.Dv.view(torch.int32))
     for a, b in ((blk.ln_dgamma, dg), (blk.ln_dbeta, db)):  # fp32 column sums in atomic order
         assert (a - b).abs().max().item() <= 1e-5 * b.abs().max().item()
