@@ -453,24 +453,52 @@ __device__ __forceinline__ void grad_dw_tile(unsigned char* smem_raw, const Tile
   });
 }
 
-// Workgroups of one launch: the weight gradients' items first (their sums are the longer chains),
-// weight by weight from w0, chunk by chunk, then computeGradDx's tiles where dX is set.
+// Items of one launch: dQw's (tile by tile, chunk by chunk), the other weights', computeGradDx's tiles
+// where dX is set. Workgroups are dealt to the 8 XCDs in turn; an XCD takes a contiguous eighth of each
+// kind (rounded up: the last ones may be empty), the weight gradients' longer sums first. (A contiguous
+// eighth of the whole list gave some XCDs only the long sums and others only computeGradDx's tiles.)
+struct GradItems {
+  int tiles, nq, nkv, nx;    // tiles of a weight; items of each kind (one list: all weights' in nq + nkv)
+  int per_q, per_kv, per_x;  // an XCD's share
+};
+__host__ __device__ inline GradItems grad_items(const TileGrad& a) {
+  GradItems g;
+  const int nb = a.C / 64;
+  g.tiles = nb * nb;
+  g.nq = a.w0 == 0 && a.w1 > 0 ? g.tiles * a.nq : 0;
+  g.nkv = g.tiles * a.nkv * (a.w1 - (a.w0 == 0 && a.w1 > 0 ? 1 : a.w0));
+  g.nx = a.dX ? (a.R + 63) / 64 * nb : 0;
+  const bool one_list = a.part && !a.dX;
+  g.per_q = (g.nq + (one_list ? g.nkv : 0) + 7) / 8;
+  g.per_kv = one_list ? 0 : (g.nkv + 7) / 8;
+  g.per_x = (g.nx + 7) / 8;
+  return g;
+}
+
 template <int NW, bool ACC>
 __global__ void __launch_bounds__(64 * NW, 2) tile_grad_kernel(TileGrad a) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[NW * kWaveLds];
-  const int item = item_of((int)blockIdx.x, (int)gridDim.x);
-  const int nb = a.C / 64, tiles = nb * nb;
-  const int nq = a.w0 == 0 && a.w1 > 0 ? tiles * a.nq : 0;                          // dQw's items
-  const int nw = nq + tiles * a.nkv * (a.w1 - (a.w0 == 0 ? min(a.w1, 1) : a.w0));  // all weights'
-  if (item < nq) {
-    const int chunk = item / tiles;
-    grad_dw_tile<NW, ACC, true>(smem_raw, a, 0, chunk, a.nq, item - chunk * tiles);
-  } else if (item < nw) {
-    const int i = (item - nq) / tiles, w = i / a.nkv;
-    grad_dw_tile<NW, ACC, false>(smem_raw, a, w + max(a.w0, 1), i - w * a.nkv, a.nkv, item - nq - i * tiles);
-  } else if (a.dX && item < nw + (a.R + 63) / 64 * nb) {
-    grad_dx_tile<NW, ACC>(smem_raw, a, item - nw);
+  const GradItems n = grad_items(a);
+  const int x = blockIdx.x & 7;
+  const int k = blockIdx.x >> 3;
+  if (k < n.per_q + n.per_kv) {
+    int item = k < n.per_q ? x * n.per_q + k : x * n.per_kv + k - n.per_q;
+    if (k < n.per_q && item < n.nq) {
+      const int chunk = item / n.tiles;
+      grad_dw_tile<NW, ACC, true>(smem_raw, a, 0, chunk, a.nq, item - chunk * n.tiles);
+      return;
+    }
+    if (k < n.per_q) {
+      if (n.per_kv) return;  // past the end of dQw's own share
+      item -= n.nq;
+    }
+    const int i = item / n.tiles, w = i / a.nkv;
+    if (item < n.nkv)
+      grad_dw_tile<NW, ACC, false>(smem_raw, a, w + max(a.w0, 1), i - w * a.nkv, a.nkv, item - i * n.tiles);
+    return;
   }
+  const int item = x * n.per_x + k - n.per_q - n.per_kv;
+  if (item < n.nx) grad_dx_tile<NW, ACC>(smem_raw, a, item);
 }
 
 // Tiles up to which a workgroup has 8 waves (one workgroup per CU); beyond it 4, two workgroups per
@@ -522,12 +550,11 @@ hipError_t launch_tile_grad(TileGrad a, float* partial, bool accumulate, hipStre
   a.nq = k.nq;
   a.nkv = k.nkv;
   a.part = k.nkv == 1 && k.nq <= 1 ? nullptr : partial;
-  const int nb = a.C / 64, tiles = nb * nb;
-  const int dw = a.w1 > a.w0 ? tiles * ((a.w0 == 0 ? k.nq : 0) + (a.w1 - std::max(a.w0, 1)) * k.nkv) : 0;
-  const unsigned grid = padded(dw + (a.dX ? (a.R + 63) / 64 * nb : 0));
+  const GradItems n = grad_items(a);
+  const unsigned grid = 8u * (unsigned)(n.per_q + n.per_kv + n.per_x);
   // computeGradDx's waves follow its own tile count alone: its sums are the same bit for bit with and
   // without weight gradients in the launch
-  const bool deep = a.dX ? (a.R + 63) / 64 * nb <= kDeepItems / 2 : grid <= kDeepItems;
+  const bool deep = a.dX ? (unsigned)n.nx <= kDeepItems / 2 : grid <= kDeepItems;
   auto kern = accumulate ? (deep ? tile_grad_kernel<8, true> : tile_grad_kernel<4, true>)
                          : (deep ? tile_grad_kernel<8, false> : tile_grad_kernel<4, false>);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(deep ? 512 : 256), 0, s, a);
