@@ -282,8 +282,10 @@ typedef struct metalllmSublayerGraph metalllmSublayerGraph;
  *            flashAttentionBackwardWorkspace, computeGradDx, computeGradDw, and
  *            castFloatToBfloat(dX) when dX_bf16 is set. dX, dQw, dKw, dVw and dProjw, which
  *            model.h zeroes before the pass and accumulates into, have one producer each here:
- *            they are written as 0 + the gradient, without being zeroed or read. When B*M and N
- *            are multiples of 128, dProjw is computed last, in computeGradDw's launch, so the
+ *            they are written as 0 + the gradient, without being zeroed or read. Where a
+ *            hand-written kernel takes computeGradDx and computeGradDw (B*M and N multiples of
+ *            128, or N a multiple of 64 and B*M*N*N at most 3e10), dProjw is computed last, in
+ *            their launch, so dOut and attn_out must last until then, and the
  *            four weight gradients are summed over other row chunks than the entry points use
  *            (equal up to fp32 summation order); every other output equals the entry points'
  *            chain bit for bit.

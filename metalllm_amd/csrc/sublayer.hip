@@ -231,6 +231,11 @@ bool tile_dw_one_ok(int R, int C) {  // projBackwarddW
 // takes them for dX, whose sums are then the same
 bool tile_dxdw_ok(int R, int C) { return R % 64 == 0 && tile_dx_ok(R, C); }
 
+// Whether two buffers of n bf16 elements do not overlap.
+bool apart(const uint16_t* a, const uint16_t* b, size_t n) {
+  return std::abs((intptr_t)(uintptr_t)a - (intptr_t)(uintptr_t)b) >= (intptr_t)(2 * n);
+}
+
 int tile_rows(const Ctx& c, const mla::TileRows& a, bool wt) {
   if (c.query) return METALLLM_ATTN_OK;
   return mla::launch_tile_rows(a, wt, c.stream) == hipSuccess ? METALLLM_ATTN_OK : METALLLM_ATTN_E_LAUNCH;
@@ -338,8 +343,8 @@ int op_qkv(const Ctx& c, const uint16_t* X, uint16_t* q, uint16_t* k, uint16_t* 
            const uint16_t* k_w, const uint16_t* v_w, int R, int C) {
   // distances in bf16 elements, from the integer addresses (the buffers may be separate allocations)
   const auto at = [](const uint16_t* ptr) { return (intptr_t)(uintptr_t)ptr; };
-  const auto apart = [&](const uint16_t* a, const uint16_t* b) { return std::abs(at(a) - at(b)) >= 2 * (intptr_t)R * C; };
-  if (tile_rows_ok(R, C, 3) && apart(q, k) && apart(k, v) && apart(q, v))
+  const size_t e = (size_t)R * C;
+  if (tile_rows_ok(R, C, 3) && apart(q, k, e) && apart(k, v, e) && apart(q, v, e))
     return tile_rows(c, mla::TileRows{X, {q_w, k_w, v_w}, {q, k, v}, 3, R, C}, false);
   const intptr_t bw = at(k_w) - at(q_w), by = at(k) - at(q);
   const intptr_t dw = bw / 2, dy = by / 2;
@@ -574,7 +579,9 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
       TRY(layernormForward(b->hidden, b->ln_xnorm, (uint16_t*)b->X, b->ln_gamma, b->ln_beta, b->ln_stdev, &lp, s));
     TRY(op_qkv(c, b->X, b->q, b->k, b->v, b->q_w, b->k_w, b->v_w, R, C));
     if (!c.query) TRY(flashAttentionForward(b->q, b->k, b->v, b->attn_out, b->l, p, s));
-    if (block && tile_rows_ok(R, C, 1)) {  // the projection's tiles add hidden as they are stored (model.h:483)
+    // the projection's tiles add hidden as they are stored (model.h:483), unless residual reuses
+    // attn_out's memory, which other tiles may still have to read
+    if (block && tile_rows_ok(R, C, 1) && apart(b->residual, b->attn_out, e)) {
       mla::TileRows t{b->attn_out, {b->proj_w}, {b->out}, 1, R, C};
       t.add = b->hidden;
       t.sum = b->residual;

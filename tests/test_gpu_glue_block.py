@@ -48,3 +48,22 @@ def test_block_ends(gpu, B, T, H, C):
     assert torch.equal(Dv.view(torch.int32), blk.Dv.view(torch.int32))
     for a, b in ((blk.ln_dgamma, dg), (blk.ln_dbeta, db)):  # fp32 column sums in atomic order
         assert (a - b).abs().max().item() <= 1e-5 * b.abs().max().item()
+
+
+def test_residual_in_attn_out(gpu):
+    """A forward pass whose residual reuses attn_out's memory: the same residual as with its own buffer
+    (the projection's tiles read rows of attn_out that other tiles' residual would have replaced)."""
+    import torch
+    import metalllm_amd.sublayer as S
+    B, T, H, C = 3, 320, 5, 320
+    rng = np.random.default_rng(7)
+    bf = lambda shape, sc=1.0, sh=0.0: to_gpu(O.f32_to_bf16((rng.standard_normal(shape) * sc + sh).astype(np.float32)), gpu)
+    blk = S.Sublayer(None, *[bf((C, C), 0.02) for _ in range(4)], H=H, hidden=bf((B, T, C), 1.0, 0.3),
+                     ln_gamma=bf((C,), 0.1, 1.0), ln_beta=bf((C,), 0.1))
+    blk.encode(0)
+    bufs = blk.buffers()
+    shared = torch.empty_like(blk.residual)
+    bufs.residual = bufs.attn_out = shared.data_ptr()
+    S.encode_phase(0, bufs, blk.p)
+    torch.cuda.synchronize()
+    assert torch.equal(shared, blk.residual)
