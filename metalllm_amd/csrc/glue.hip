@@ -191,16 +191,26 @@ __global__ void __launch_bounds__(256) ln_fwd_kernel(const uint16_t* __restrict_
   }
 }
 
+// How ln_bwd_kernel's steps (16/S rows each) are dealt to its workgroups. q = 0: step k of workgroup
+// b is k*gridDim.x + b. Else contiguous ranges of about q steps, the first `more` workgroups one more,
+// and of each three workgroups one has a step less and one a step more (ln_bwd_deal says when).
+struct LnDeal {
+  uint32_t q, more;
+};
+__device__ __forceinline__ uint32_t ln_first_step(const LnDeal& d, uint32_t b) {
+  return b * d.q + min(b, d.more) - (b % 3 ? 1u : 0u);
+}
+
 // layernorm.metal:73-127. A workgroup of 16 waves takes 16/S rows at a time, each by S waves (S > 1
 // for rows of more than 1024 columns, so that a lane holds at most two 16-byte chunks of a row: with
-// whole wide rows per lane the sums and the row leave room for one wave per SIMD). Row r of the
-// workgroup's k-th step is (k*gridDim.x + blockIdx.x)*16/S + r. Each lane keeps the dgamma/dbeta
+// whole wide rows per lane the sums and the row leave room for one wave per SIMD), in the steps
+// that LnDeal says. Each lane keeps the dgamma/dbeta
 // partial sums of its own columns across its rows; the waves' partials meet in LDS and one fp32
 // atomic per column adds the workgroup's sum. All workgroups add into the same 2*cols addresses and
 // atomics on one address run one after another (about 34 ns each), so the grid is a compromise
 // (ln_bwd_grid). Four waves a workgroup, up to 1024 workgroups, rounding in integer arithmetic and
 // row sums through LDS permutes took 48 us at 16384 x 768, 71 us at 32768 x 1024 and 85 us at 4096 x
-// 4096; this takes 24, 35 (5.8 TB/s) and 24 us.
+// 4096; this takes 19, 35 (5.8 TB/s) and 22 us (the first and last 22 and 24 before LnDeal's ranges).
 // BLOCK (the phase encoder's form): the gradient comes in as the fp32 dX and is rounded to bf16
 // first (castFloatToBfloat), and `add` is added to the result, rounded again (residualAdd): the
 // three kernels' results bit for bit, with one read of dX and one write of dZ instead of three and
@@ -212,7 +222,7 @@ __global__ void __launch_bounds__(1024) ln_bwd_kernel(uint16_t* __restrict__ dZ,
                                                       const uint16_t* __restrict__ gamma,
                                                       const float* __restrict__ stdev, uint16_t* __restrict__ dxnorm,
                                                       float* __restrict__ dgamma, float* __restrict__ dbeta,
-                                                      uint32_t rows, uint32_t cols) {
+                                                      uint32_t rows, uint32_t cols, LnDeal deal) {
   constexpr int W = 16, RW = W / S;  // waves, rows per step
   __shared__ float red[2][W][512];
   __shared__ float2 rsum[2][W];  // S > 1: the waves' parts of a row's two sums, by step parity
@@ -231,7 +241,10 @@ __global__ void __launch_bounds__(1024) ln_bwd_kernel(uint16_t* __restrict__ dZ,
     gam[j] = c < nchunk ? ((const uint4*)gamma)[c] : uint4{0u, 0u, 0u, 0u};
   }
   const uint4 none = uint4{0u, 0u, 0u, 0u};
-  for (uint32_t r0 = blockIdx.x * RW, it = 0; r0 < rows; r0 += RW * gridDim.x, ++it) {
+  const uint32_t first = deal.q ? ln_first_step(deal, blockIdx.x) : blockIdx.x, stride = deal.q ? 1 : gridDim.x;
+  const uint32_t end = deal.q && blockIdx.x + 1 < gridDim.x ? ln_first_step(deal, blockIdx.x + 1) : (rows + RW - 1) / RW;
+  for (uint32_t at = first, it = 0; at < end; at += stride, ++it) {
+    const uint32_t r0 = at * RW;
     const uint32_t row = r0 + rg;
     const bool live = row < rows;  // false only past the last row: the wave adds zeros and stores nothing
     const size_t base = (size_t)min(row, rows - 1) * cols;
@@ -348,6 +361,19 @@ uint32_t ln_bwd_grid(uint32_t rows, uint32_t cols, int rows_per_step) {
   return std::max<uint32_t>(1, std::min<uint32_t>(steps, std::min<uint32_t>(256, std::max<uint32_t>(n, 16))));
 }
 
+// Equally long workgroups all end, and add into the same columns, at the same time. With ends a step
+// apart one third's atomics run while the others still stream rows: 16384 x 768 22.3 -> 19.4 us, 12288
+// x 768 19.3 -> 16.8, 8192 x 1536 23.6 -> 20.1, 32768 x 384 21.8 -> 20.6. Not with fewer than three
+// steps each; nor where a step is long against the atomics and the ends drift apart by themselves
+// (98304 elements a workgroup, 24576 x 1024, 28.8 -> 28.4; 131072, 32768 x 1024, 34.5 -> 35.6); nor
+// where the steps do not divide and are few, so that ends differ already (13000 x 520, three and a
+// third steps, 17.1 -> 17.0, the encoder's form 21.1 -> 22.1; 32768 x 200, eight and a half, 20.4 -> 19.6).
+LnDeal ln_bwd_deal(uint32_t rows, uint32_t cols, int rows_per_step, uint32_t n) {
+  const uint32_t steps = (rows + rows_per_step - 1) / rows_per_step, q = steps / n, more = steps - q * n;
+  const bool apart = q >= 3 && (uint64_t)rows * cols < 100000ull * n && (q >= 8 || more * 8 < n);
+  return apart ? LnDeal{q, more} : LnDeal{0, 0};
+}
+
 template <bool BLOCK>
 hipError_t launch_ln_bwd(uint16_t* dZ, const float* dX, const uint16_t* add, const uint16_t* xnorm, const uint16_t* gamma,
                          const float* stdev, uint16_t* dxnorm, float* dgamma, float* dbeta, uint32_t rows, uint32_t cols,
@@ -355,9 +381,10 @@ hipError_t launch_ln_bwd(uint16_t* dZ, const float* dX, const uint16_t* add, con
   const int nch = (int)((cols / 8 + 63) / 64);
   const int S = nch <= 2 ? 1 : (nch <= 4 ? 2 : 4);
   const dim3 grid(ln_bwd_grid(rows, cols, 16 / S));
+  const LnDeal deal = ln_bwd_deal(rows, cols, 16 / S, grid.x);
 #define LNB(NC, S_) \
   hipLaunchKernelGGL((ln_bwd_kernel<NC, S_, BLOCK>), grid, dim3(1024), 0, s, dZ, dX, add, xnorm, gamma, stdev, dxnorm, \
-                     dgamma, dbeta, rows, cols)
+                     dgamma, dbeta, rows, cols, deal)
   if (nch == 1) LNB(1, 1);
   else if (S == 1) LNB(2, 1);
   else if (S == 2) LNB(2, 2);

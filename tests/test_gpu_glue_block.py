@@ -12,7 +12,9 @@ from tests.attn_case import to_gpu
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("rows,cols", [(4099, 1032), (1000, 1536), (515, 2056), (33, 3080), (1, 1024), (17, 512)])
+@pytest.mark.parametrize("rows,cols", [(4099, 1032), (1000, 1536), (515, 2056), (33, 3080), (1, 1024), (17, 512),
+                                       # workgroups whose ranges of steps differ by one (ln_bwd_deal)
+                                       (3077, 4096), (12281, 64), (12288, 768)])
 def test_layernorm_row_split(gpu, rows, cols):
     import metalllm_amd.glue as G
     glue_checks.test_layernorm_forward_backward(gpu, G, rows, cols, 1.0)
