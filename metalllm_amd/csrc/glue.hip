@@ -210,7 +210,8 @@ __device__ __forceinline__ uint32_t ln_first_step(const LnDeal& d, uint32_t b) {
 // atomics on one address run one after another (about 34 ns each), so the grid is a compromise
 // (ln_bwd_grid). Four waves a workgroup, up to 1024 workgroups, rounding in integer arithmetic and
 // row sums through LDS permutes took 48 us at 16384 x 768, 71 us at 32768 x 1024 and 85 us at 4096 x
-// 4096; this takes 19, 35 (5.8 TB/s) and 22 us (the first and last 22 and 24 before LnDeal's ranges).
+// 4096; this took 24, 35 (5.8 TB/s) and 24 us, and LnDeal's ranges take the first and last another 13
+// and 8% down (back to back 22.3 -> 19.4 and 29.9 -> 27.5 us).
 // BLOCK (the phase encoder's form): the gradient comes in as the fp32 dX and is rounded to bf16
 // first (castFloatToBfloat), and `add` is added to the result, rounded again (residualAdd): the
 // three kernels' results bit for bit, with one read of dX and one write of dZ instead of three and
