@@ -24,12 +24,12 @@
 #include <rocblas/rocblas.h>
 
 #include <algorithm>
-#include <cstdlib>
 #include <mutex>
 #include <vector>
 
 #include "../../include/metalllm_attn.h"
 #include "attn_launch.hpp"
+#include "overlap.hpp"
 #include "sublayer_tile.hpp"
 
 namespace mla {  // glue.hip
@@ -231,9 +231,39 @@ bool tile_dw_one_ok(int R, int C) {  // projBackwarddW
 // takes them for dX, whose sums are then the same
 bool tile_dxdw_ok(int R, int C) { return R % 64 == 0 && tile_dx_ok(R, C); }
 
-// Whether two buffers of n bf16 elements do not overlap.
-bool apart(const uint16_t* a, const uint16_t* b, size_t n) {
-  return std::abs((intptr_t)(uintptr_t)a - (intptr_t)(uintptr_t)b) >= (intptr_t)(2 * n);
+// n bf16 or fp32 elements
+mla::Span span(const uint16_t* p, size_t n) { return {p, 2 * n}; }
+mla::Span span(const float* p, size_t n) { return {p, 4 * n}; }
+
+// Whether the products' destinations are apart from each other and from what any of the products
+// reads. The tile kernels need that: their workgroups, of one product or of several in one launch,
+// read operands while others store. The calls in turn, which they replace, do not always: the library
+// path of the gradient products reads the fp32 dQ once, into its split, before anything is written,
+// adds dKw and dVw one after the other, and writes a weight gradient when its sums are complete.
+bool qkv_apart(const uint16_t* X, const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* q_w,
+               const uint16_t* k_w, const uint16_t* v_w, int R, int C) {
+  const size_t e = (size_t)R * C, w = (size_t)C * C;
+  return !mla::any_overlap({span(q, e), span(k, e), span(v, e)}) &&
+         !mla::any_overlap({span(q, e), span(k, e), span(v, e)}, {span(X, e), span(q_w, w), span(k_w, w), span(v_w, w)});
+}
+bool rows_apart(const uint16_t* x, const uint16_t* w, const uint16_t* y, int R, int C) {
+  const size_t e = (size_t)R * C;
+  return !mla::any_overlap({span(y, e)}, {span(x, e), span(w, (size_t)C * C)});
+}
+bool proj_dw_apart(const uint16_t* attn_out, const uint16_t* dZ, const uint16_t* dProjw, int R, int C) {
+  const size_t e = (size_t)R * C;
+  return !mla::any_overlap({span(dProjw, (size_t)C * C)}, {span(attn_out, e), span(dZ, e)});
+}
+bool grad_dx_apart(const float* dX, const uint16_t* qw, const uint16_t* kw, const uint16_t* vw, const float* dQ,
+                   const uint16_t* dK, const uint16_t* dV, int R, int C) {
+  const size_t e = (size_t)R * C, w = (size_t)C * C;
+  return !mla::any_overlap({span(dX, e)}, {span(dQ, e), span(dK, e), span(dV, e), span(qw, w), span(kw, w), span(vw, w)});
+}
+bool grad_dw_apart(const uint16_t* x, const float* dQ, const uint16_t* dK, const uint16_t* dV, const float* dQw,
+                   const uint16_t* dKw, const uint16_t* dVw, int R, int C) {
+  const size_t e = (size_t)R * C, w = (size_t)C * C;
+  return !mla::any_overlap({span(dQw, w), span(dKw, w), span(dVw, w)}) &&
+         !mla::any_overlap({span(dQw, w), span(dKw, w), span(dVw, w)}, {span(x, e), span(dQ, e), span(dK, e), span(dV, e)});
 }
 
 int tile_rows(const Ctx& c, const mla::TileRows& a, bool wt) {
@@ -259,24 +289,26 @@ int row_chunks(int R) {
 
 // Elements of the dQ split (hi, then lo) that the library paths of computeGradDx (dx) and
 // computeGradDw read: none where the hand-written kernels take the shape (they split in registers).
-size_t split_need(int R, int C, bool dx) {
-  const bool ok = dx ? tile_dx_ok(R, C) || mla::grad_dx_fused_ok(R, C) : tile_dw_ok(R, C) || mla::grad_dw_fused_ok(R, C);
+// `tiles`: the buffers allow the tile kernels (the *_apart conditions).
+size_t split_need(int R, int C, bool dx, bool tiles) {
+  const bool ok = dx ? (tiles && tile_dx_ok(R, C)) || mla::grad_dx_fused_ok(R, C)
+                     : (tiles && tile_dw_ok(R, C)) || mla::grad_dw_fused_ok(R, C);
   return ok ? 0 : 2 * (size_t)R * C;
 }
 
 // fp32 partial floats for projBackwarddW, computeGradDw and the encoder's launch: the hand-written
 // kernels' chunks, or row_chunks(R) products of C x C (twice that for computeGradDw's dQw) on the
 // library path.
-size_t partial_need(int R, int C) {
+size_t partial_need(int R, int C, bool tiles) {
   const size_t tile = C % 64 || R % 64 ? 0
                                        : std::max({mla::tile_grad_partial_floats(R, C, 3, 4, false),
                                                    mla::tile_grad_partial_floats(R, C, 0, 3, false),
                                                    mla::tile_grad_partial_floats(R, C, 0, 4, true)});
-  if (tile_dw_one_ok(R, C) && tile_dw_ok(R, C) && tile_dxdw_ok(R, C)) return tile;
+  if (tiles && tile_dw_one_ok(R, C) && tile_dw_ok(R, C) && tile_dxdw_ok(R, C)) return tile;
   if (mla::grad_dw_fused_ok(R, C))
     return std::max({tile, mla::grad_dw_one_partial_floats(R, C), mla::grad_dw_partial_floats(R, C),
                      mla::grad_dw4_partial_floats(R, C)});
-  return 2 * (size_t)row_chunks(R) * C * C;
+  return std::max(tile, 2 * (size_t)row_chunks(R) * C * C);
 }
 
 int xt_g_partials(const Ctx& c, const uint16_t* X, const uint16_t* G, int R, int C, int parts, float* out) {
@@ -343,8 +375,7 @@ int op_qkv(const Ctx& c, const uint16_t* X, uint16_t* q, uint16_t* k, uint16_t* 
            const uint16_t* k_w, const uint16_t* v_w, int R, int C) {
   // distances in bf16 elements, from the integer addresses (the buffers may be separate allocations)
   const auto at = [](const uint16_t* ptr) { return (intptr_t)(uintptr_t)ptr; };
-  const size_t e = (size_t)R * C;
-  if (tile_rows_ok(R, C, 3) && apart(q, k, e) && apart(k, v, e) && apart(q, v, e))
+  if (tile_rows_ok(R, C, 3) && qkv_apart(X, q, k, v, q_w, k_w, v_w, R, C))
     return tile_rows(c, mla::TileRows{X, {q_w, k_w, v_w}, {q, k, v}, 3, R, C}, false);
   const intptr_t bw = at(k_w) - at(q_w), by = at(k) - at(q);
   const intptr_t dw = bw / 2, dy = by / 2;
@@ -364,16 +395,17 @@ int op_qkv(const Ctx& c, const uint16_t* X, uint16_t* q, uint16_t* k, uint16_t* 
 }
 
 int op_proj_fwd(const Ctx& c, const uint16_t* attn_out, const uint16_t* proj_w, uint16_t* out, int R, int C) {
-  if (tile_rows_ok(R, C, 1)) return tile_rows(c, mla::TileRows{attn_out, {proj_w}, {out}, 1, R, C}, false);
+  if (tile_rows_ok(R, C, 1) && rows_apart(attn_out, proj_w, out, R, C))
+    return tile_rows(c, mla::TileRows{attn_out, {proj_w}, {out}, 1, R, C}, false);
   return gemm_rm(c, false, false, R, C, C, attn_out, BF, C, proj_w, BF, C, 0.0f, out, BF, C);
 }
 
-// partial: at least partial_need(R, C) floats. accumulate = false: dProjw is written as if it
+// partial: at least partial_need(R, C, proj_dw_apart) floats. accumulate = false: dProjw is written as if it
 // held zeros (the phase encoder; every op_* below takes the same flag). Larger products in multiples
 // of 128 run computeGradDw's 128-wide kernel (sublayer_gemm.hip) on the one bf16 gradient.
 int op_proj_dw(const Ctx& c, const uint16_t* attn_out, const uint16_t* dZ, uint16_t* dProjw, int R, int C,
                float* partial, bool accumulate = true) {
-  if (tile_dw_one_ok(R, C)) {
+  if (tile_dw_one_ok(R, C) && proj_dw_apart(attn_out, dZ, dProjw, R, C)) {
     mla::TileGrad a{};
     a.x[3] = attn_out, a.g[3] = dZ, a.dW[3] = dProjw, a.w0 = 3, a.w1 = 4, a.R = R, a.C = C;
     return tile_grad(c, a, partial, accumulate);
@@ -390,16 +422,17 @@ int op_proj_dw(const Ctx& c, const uint16_t* attn_out, const uint16_t* dZ, uint1
 }
 
 int op_proj_dx(const Ctx& c, const uint16_t* dZ, const uint16_t* proj_w, uint16_t* dAttn, int R, int C) {
-  if (tile_rows_ok(R, C, 1)) return tile_rows(c, mla::TileRows{dZ, {proj_w}, {dAttn}, 1, R, C}, true);
+  if (tile_rows_ok(R, C, 1) && rows_apart(dZ, proj_w, dAttn, R, C))
+    return tile_rows(c, mla::TileRows{dZ, {proj_w}, {dAttn}, 1, R, C}, true);
   return gemm_rm(c, false, true, R, C, C, dZ, BF, C, proj_w, BF, C, 0.0f, dAttn, BF, C);
 }
 
 // The hand-written kernels read the fp32 dQ themselves; the library runs on hi, lo, the two-term bf16
-// split of dQ (split_dq).
+// split of dQ (split_dq). tiles: the buffers allow the tile kernel (grad_dx_apart).
 int op_grad_dx(const Ctx& c, float* dX, const uint16_t* qw, const uint16_t* kw, const uint16_t* vw, const float* dQ,
-               const uint16_t* hi, const uint16_t* lo, const uint16_t* dK, const uint16_t* dV, int R, int C,
+               const uint16_t* hi, const uint16_t* lo, const uint16_t* dK, const uint16_t* dV, int R, int C, bool tiles,
                bool accumulate = true) {
-  if (tile_dx_ok(R, C))
+  if (tiles && tile_dx_ok(R, C))
     return tile_grad(c, mla::TileGrad{dX, dQ, {qw, kw, vw}, {}, {nullptr, dK, dV}, {}, 0, 0, R, C}, nullptr, accumulate);
   if (mla::grad_dx_fused_ok(R, C)) {
     if (c.query) return METALLLM_ATTN_OK;
@@ -413,11 +446,11 @@ int op_grad_dx(const Ctx& c, float* dX, const uint16_t* qw, const uint16_t* kw, 
   return gemm_rm(c, false, true, R, C, C, dV, BF, C, vw, BF, C, 1.0f, dX, F32, C);
 }
 
-// partial: at least partial_need(R, C) floats; hi, lo as in op_grad_dx.
+// partial: at least partial_need(R, C, tiles) floats; hi, lo as in op_grad_dx; tiles: grad_dw_apart.
 int op_grad_dw(const Ctx& c, const uint16_t* x, const float* dQ, const uint16_t* hi, const uint16_t* lo,
                const uint16_t* dK, const uint16_t* dV, float* dQw, uint16_t* dKw, uint16_t* dVw, int R, int C,
-               float* part, bool accumulate = true) {
-  if (tile_dw_ok(R, C))
+               float* part, bool tiles, bool accumulate = true) {
+  if (tiles && tile_dw_ok(R, C))
     return tile_grad(c, mla::TileGrad{nullptr, dQ, {}, {x, x, x}, {nullptr, dK, dV}, {dQw, dKw, dVw}, 0, 3, R, C}, part,
                      accumulate);
   if (mla::grad_dw_fused_ok(R, C)) {
@@ -477,7 +510,8 @@ int projBackwarddW(const uint16_t* attn_out, const uint16_t* dZ, uint16_t* dProj
   const int R = (int)(p->B * p->M), C = (int)p->N;
   Public u(stream);
   TRY(u.s.rc);
-  TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial_need(R, C), u.c.stream));
+  const size_t partial = partial_need(R, C, proj_dw_apart(attn_out, dZ, dProjw, R, C));
+  TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial, u.c.stream));
   return op_proj_dw(u.c, attn_out, dZ, dProjw, R, C, u.s.st->partial);
 }
 
@@ -498,10 +532,11 @@ int computeGradDx(float* dX, const uint16_t* qw, const uint16_t* kw, const uint1
   const size_t e = (size_t)R * C;
   Public u(stream);
   TRY(u.s.rc);
-  if (!split_need(R, C, true)) return op_grad_dx(u.c, dX, qw, kw, vw, dQ, nullptr, nullptr, dK, dV, R, C);
+  const bool tiles = grad_dx_apart(dX, qw, kw, vw, dQ, dK, dV, R, C);
+  if (!split_need(R, C, true, tiles)) return op_grad_dx(u.c, dX, qw, kw, vw, dQ, nullptr, nullptr, dK, dV, R, C, tiles);
   TRY(ensure(u.s.st->split, u.s.st->split_elems, 2 * e, u.c.stream));
   TRY(split_dq(u.c, dQ, e, u.s.st->split));
-  return op_grad_dx(u.c, dX, qw, kw, vw, dQ, u.s.st->split, u.s.st->split + e, dK, dV, R, C);
+  return op_grad_dx(u.c, dX, qw, kw, vw, dQ, u.s.st->split, u.s.st->split + e, dK, dV, R, C, tiles);
 }
 
 int computeGradDw(const uint16_t* x, const float* dQ, const uint16_t* dK, const uint16_t* dV, float* dQw,
@@ -512,12 +547,14 @@ int computeGradDw(const uint16_t* x, const float* dQ, const uint16_t* dK, const 
   const size_t e = (size_t)R * C;
   Public u(stream);
   TRY(u.s.rc);
-  TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial_need(R, C), u.c.stream));
-  if (!split_need(R, C, false))
-    return op_grad_dw(u.c, x, dQ, nullptr, nullptr, dK, dV, dQw, dKw, dVw, R, C, u.s.st->partial);
+  const bool tiles = grad_dw_apart(x, dQ, dK, dV, dQw, dKw, dVw, R, C);
+  TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial_need(R, C, tiles), u.c.stream));
+  if (!split_need(R, C, false, tiles))
+    return op_grad_dw(u.c, x, dQ, nullptr, nullptr, dK, dV, dQw, dKw, dVw, R, C, u.s.st->partial, tiles);
   TRY(ensure(u.s.st->split, u.s.st->split_elems, 2 * e, u.c.stream));
   TRY(split_dq(u.c, dQ, e, u.s.st->split));
-  return op_grad_dw(u.c, x, dQ, u.s.st->split, u.s.st->split + e, dK, dV, dQw, dKw, dVw, R, C, u.s.st->partial);
+  return op_grad_dw(u.c, x, dQ, u.s.st->split, u.s.st->split + e, dK, dV, dQw, dKw, dVw, R, C, u.s.st->partial,
+                    tiles);
 }
 
 }  // extern "C"
@@ -581,7 +618,7 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
     if (!c.query) TRY(flashAttentionForward(b->q, b->k, b->v, b->attn_out, b->l, p, s));
     // the projection's tiles add hidden as they are stored (model.h:483), unless residual reuses
     // attn_out's memory, which other tiles may still have to read
-    if (block && tile_rows_ok(R, C, 1) && apart(b->residual, b->attn_out, e)) {
+    if (block && tile_rows_ok(R, C, 1) && !mla::any_overlap({span(b->residual, e)}, {span(b->attn_out, e)})) {
       mla::TileRows t{b->attn_out, {b->proj_w}, {b->out}, 1, R, C};
       t.add = b->hidden;
       t.sum = b->residual;
@@ -628,7 +665,7 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
                                         attn_ws_bytes, p, s));
   }
   uint16_t* lo = nullptr;  // no split when both hand-written kernels take the shape
-  if (!tile && std::max(split_need(R, C, true), split_need(R, C, false))) {
+  if (!tile && std::max(split_need(R, C, true, true), split_need(R, C, false, true))) {
     TRY(split_dq(c, b->dQ, e, split));  // one split serves both consumers
     lo = split + e;
   } else {
@@ -645,8 +682,8 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
                                            c.stream) != hipSuccess)
       return METALLLM_ATTN_E_LAUNCH;
   } else {
-    TRY(op_grad_dx(c, b->dX, b->q_w, b->k_w, b->v_w, b->dQ, split, lo, b->dK, b->dV, R, C, false));
-    TRY(op_grad_dw(c, b->X, b->dQ, split, lo, b->dK, b->dV, b->dQw, b->dKw, b->dVw, R, C, partial, false));
+    TRY(op_grad_dx(c, b->dX, b->q_w, b->k_w, b->v_w, b->dQ, split, lo, b->dK, b->dV, R, C, true, false));
+    TRY(op_grad_dw(c, b->X, b->dQ, split, lo, b->dK, b->dV, b->dQw, b->dKw, b->dVw, R, C, partial, true, false));
   }
   if (c.query) return METALLLM_ATTN_OK;
   if (block)  // model.h:692-695: cast of dX, ln1 backward and the skip add
@@ -665,9 +702,9 @@ int build_graph(metalllmSublayerGraph* g, const metalllmSublayerBuffers* b, cons
     return METALLLM_ATTN_E_LIBRARY;
   }
   if (g->phase == 1) {
-    const size_t split = std::max(split_need(R, C, true), split_need(R, C, false));
+    const size_t split = std::max(split_need(R, C, true, true), split_need(R, C, false, true));
     if (split && hipMalloc((void**)&g->split, split * sizeof(uint16_t)) != hipSuccess) g->split = nullptr;
-    const size_t partial = partial_need(R, C);
+    const size_t partial = partial_need(R, C, true);
     if (partial && hipMalloc((void**)&g->partial, partial * sizeof(float)) != hipSuccess) g->partial = nullptr;
     TRY(metalllmAttnBackwardWorkspaceSize(p, &g->attn_ws_bytes));
     if (hipMalloc(&g->attn_ws, g->attn_ws_bytes) != hipSuccess) g->attn_ws = nullptr;
@@ -716,8 +753,9 @@ int metalllmSublayerEncode(int phase, const metalllmSublayerBuffers* b, const At
   TRY(u.s.rc);
   uint64_t ws = 0;
   if (phase == 1) {
-    TRY(ensure(u.s.st->split, u.s.st->split_elems, std::max(split_need(R, C, true), split_need(R, C, false)), u.c.stream));
-    TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial_need(R, C), u.c.stream));
+    TRY(ensure(u.s.st->split, u.s.st->split_elems, std::max(split_need(R, C, true, true), split_need(R, C, false, true)),
+               u.c.stream));
+    TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial_need(R, C, true), u.c.stream));
     TRY(metalllmAttnBackwardWorkspaceSize(p, &ws));
     TRY(ensure(u.s.st->attn_ws, u.s.st->attn_ws_bytes, (size_t)ws, u.c.stream));
   }
@@ -735,7 +773,7 @@ int metalllmSublayerReserve(const AttentionParams* p) {
   TRY(u.s.rc);
   // what the library path of this shape would take too: a smaller shape may run it
   const bool lib = !mla::grad_dw_fused_ok(R, C);
-  const size_t partial = std::max(partial_need(R, C), lib ? 2 * (size_t)row_chunks(R) * C * C : 0);
+  const size_t partial = std::max(partial_need(R, C, true), lib ? 2 * (size_t)row_chunks(R) * C * C : 0);
   TRY(ensure(u.s.st->split, u.s.st->split_elems, lib ? 2 * (size_t)R * C : 0, nullptr));
   TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial, nullptr));
   TRY(ensure(u.s.st->attn_ws, u.s.st->attn_ws_bytes, (size_t)ws, nullptr));
