@@ -285,10 +285,13 @@ typedef struct metalllmSublayerGraph metalllmSublayerGraph;
  *            they are written as 0 + the gradient, without being zeroed or read. Where a
  *            hand-written kernel takes computeGradDx and computeGradDw (B*M and N multiples of
  *            128, or N a multiple of 64 and B*M*N*N at most 3e10), dProjw is computed last, in
- *            their launch, so dOut and attn_out must last until then, and the
- *            four weight gradients are summed over other row chunks than the entry points use
- *            (equal up to fp32 summation order); every other output equals the entry points'
- *            chain bit for bit.
+ *            their launch, and the four weight gradients are summed over other row chunks than the
+ *            entry points use (equal up to fp32 summation order); every other output equals the
+ *            entry points' chain bit for bit.
+ * Buffers may share memory as that order allows: an output may lie in the memory of a buffer that no
+ * later call of the phase reads (dK, dV or dQ in attn_out's or, for the sublayer alone, dOut's; Dsum
+ * in dOut's; residual in attn_out's). Where they do, the calls that a joint launch would replace run
+ * one after another, dProjw first among them.
  * With the block fields set: phase 0 starts with layernormForward(hidden -> X) and ends with
  * residualAdd(hidden, out -> residual); phase 1 also zeroes ln_dgamma/ln_dbeta, casts dX into
  * dStream, then runs layernormBackward(dStream) and residualAdd(dStream, dOut -> dStream).
@@ -325,6 +328,13 @@ int metalllmAttnBackwardPart(int part, const uint16_t* dZ, const float* d, const
                              const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
                              void* workspace, uint64_t workspace_bytes, const AttentionParams* p,
                              metalllm_stream_t stream);
+
+/* Test hook (no counterpart in the reference): which dispatches a phase joins in one launch for these
+ * buffers and this shape, as bits. Phase 0: 1 = residualAdd in projForward's launch. Phase 1: 1 =
+ * computeD in projBackwarddX's, 2 = dProjw last, with the other weight gradients, 4 = the gradient
+ * products' buffers are apart, as their kernels on 64 x 64 tiles need. Negative error codes as
+ * metalllmSublayerEncode. Host-only: nothing is read through the pointers. */
+int metalllmSublayerRoute(int phase, const metalllmSublayerBuffers* b, const AttentionParams* p);
 
 /* Static description of an error code (no counterpart in the reference, which has no error
  * path per kernel; model.h:333-336,361-365 only print). */

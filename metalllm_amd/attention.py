@@ -30,7 +30,8 @@ EXPORTED = ("flashAttentionForward", "computeD", "flashAttentionBackward", "meta
             "flashAttentionBackwardWorkspace", "metalllmAttnBackwardWorkspaceSize", "residualAdd",
             "layernormForward", "layernormBackward",
             "metalllmSublayerGraphCreate", "metalllmSublayerGraphLaunch", "metalllmSublayerGraphDestroy",
-            "metalllmSublayerReserve", "flashAttentionBackwardNoAlloc", "metalllmAttnForwardItems")
+            "metalllmSublayerReserve", "flashAttentionBackwardNoAlloc", "metalllmAttnForwardItems",
+            "metalllmSublayerRoute")
 NOALLOC_SCRATCH_BYTES = 64 << 20  # METALLLM_ATTN_NOALLOC_SCRATCH_BYTES
 
 

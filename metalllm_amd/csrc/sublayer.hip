@@ -603,6 +603,44 @@ int check_phase(int phase, const metalllmSublayerBuffers* b, const AttentionPara
   return METALLLM_ATTN_OK;
 }
 
+// Which of a phase's dispatches go into one launch: by shape, and where the buffers that the launch
+// would read and write in no order are apart. A buffer may otherwise reuse the memory of one that the
+// phase has finished with in the reference's order (dK in attn_out's, Dsum in dOut's, residual in
+// attn_out's).
+struct Joins {
+  bool residual;  // phase 0: residualAdd in projForward's tiles
+  bool d;         // phase 1: computeD and the zeroing of the layernorm gradients in projBackwarddX's tiles
+  bool dprojw;    // phase 1: dProjw last, with the other weight gradients
+  bool tiles;     // phase 1: the gradient products' buffers allow the tile kernels
+};
+Joins joins(int phase, const metalllmSublayerBuffers* b, const AttentionParams* p) {
+  const int R = (int)(p->B * p->M), C = (int)p->N;
+  const size_t e = (size_t)R * C, w = (size_t)C * C;
+  using mla::any_overlap;
+  const mla::Span attn_out = span(b->attn_out, e), proj_w = span(b->proj_w, w);
+  Joins j{};
+  if (phase == 0) {
+    j.residual = b->hidden && tile_rows_ok(R, C, 1) && rows_apart(b->attn_out, b->proj_w, b->out, R, C) &&
+                 !any_overlap({span(b->residual, e)}, {attn_out, proj_w});
+    return j;
+  }
+  const mla::Span X = span(b->X, e), dOut = span(b->dOut, e), Dsum = span(b->Dsum, (size_t)R * p->NH), dX = span(b->dX, e);
+  const mla::Span dQ = span(b->dQ, e), dK = span(b->dK, e), dV = span(b->dV, e);
+  const mla::Span dWq = span(b->dQw, w), dWk = span(b->dKw, w), dWv = span(b->dVw, w), dWp = span(b->dProjw, w);
+  j.d = p->D == 64 && tile_rows_ok(R, C, 1) && rows_apart(b->dOut, b->proj_w, b->dAttn, R, C) &&
+        !any_overlap({Dsum}, {dOut, proj_w});
+  j.tiles = grad_dx_apart(b->dX, b->q_w, b->k_w, b->v_w, b->dQ, b->dK, b->dV, R, C) &&
+            grad_dw_apart(b->X, b->dQ, b->dK, b->dV, b->dQw, b->dKw, b->dVw, R, C) &&
+            !any_overlap({dX, dWq, dWk, dWv, dWp}) &&
+            !any_overlap({dWq, dWk, dWv, dWp}, {span(b->q_w, w), span(b->k_w, w), span(b->v_w, w), attn_out, dOut}) &&
+            !any_overlap({dX}, {X}) && !any_overlap({dWp}, {X, dQ, dK, dV});
+  // dProjw reads attn_out and dOut: at the end only where nothing the phase writes before that, nor
+  // dX in the same launch, replaces them
+  j.dprojw = ((j.tiles && tile_dxdw_ok(R, C)) || (mla::grad_dw_fused_ok(R, C) && mla::grad_dx_fused_ok(R, C))) &&
+             !any_overlap({span(b->dAttn, e), Dsum, dQ, dK, dV, dX}, {attn_out, dOut});
+  return j;
+}
+
 // The launch sequence of one phase (model.h:444-483 forward, :549-555 and :620-693 backward).
 int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const AttentionParams* p, uint16_t* split,
            float* partial, void* attn_ws, uint64_t attn_ws_bytes) {
@@ -611,14 +649,13 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
   const metalllm_stream_t s = (metalllm_stream_t)c.stream;
   const bool block = b->hidden != nullptr;
   const LayernormParams lp{(uint32_t)R, (uint32_t)C, (uint32_t)std::min(C, 1024), b->ln_eps};
+  const Joins j = joins(phase, b, p);
   if (phase == 0) {
     if (block && !c.query)  // model.h:445: X = ln1(hidden)
       TRY(layernormForward(b->hidden, b->ln_xnorm, (uint16_t*)b->X, b->ln_gamma, b->ln_beta, b->ln_stdev, &lp, s));
     TRY(op_qkv(c, b->X, b->q, b->k, b->v, b->q_w, b->k_w, b->v_w, R, C));
     if (!c.query) TRY(flashAttentionForward(b->q, b->k, b->v, b->attn_out, b->l, p, s));
-    // the projection's tiles add hidden as they are stored (model.h:483), unless residual reuses
-    // attn_out's memory, which other tiles may still have to read
-    if (block && tile_rows_ok(R, C, 1) && !mla::any_overlap({span(b->residual, e)}, {span(b->attn_out, e)})) {
+    if (j.residual) {  // the projection's tiles add hidden as they are stored (model.h:483)
       mla::TileRows t{b->attn_out, {b->proj_w}, {b->out}, 1, R, C};
       t.add = b->hidden;
       t.sum = b->residual;
@@ -633,18 +670,17 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
   // runs them in write mode instead: the result is bit for bit 0 + the gradient (-0 becomes +0),
   // without the zeroing pass and without reading the destinations. The attention backward writes
   // dQ, dK and dV in full; the block's layernorm gradients (model.h:545-546), which its backward
-  // adds into with atomics, are zeroed by computeD's launch.
-  // With the hand-written weight-gradient kernel, dProjw (which nothing in this phase reads) is
-  // computed at the end, as a fourth weight of computeGradDw's launch and reduction: one launch of
-  // balanced items instead of projBackwarddW's own short-item launch. Its sum then runs over
-  // other row chunks than the entry point's, so it can differ from projBackwarddW's result by the
-  // fp32 summation order (one bf16 rounding step at most).
-  const bool tile = tile_dxdw_ok(R, C);
-  const bool fuse_pdw = tile || (mla::grad_dw_fused_ok(R, C) && mla::grad_dx_fused_ok(R, C));
-  if (!fuse_pdw) TRY(op_proj_dw(c, b->attn_out, b->dOut, b->dProjw, R, C, partial, false));
+  // adds into with atomics, are zeroed by the launch that computes D (projBackwarddX's tiles, or
+  // computeD's).
+  // dProjw (which nothing in this phase reads) joins computeGradDw's launch at the end as a fourth
+  // weight: one launch of balanced items instead of projBackwarddW's own short-item launch. Its sum
+  // then runs over other row chunks than the entry point's, so it can differ from projBackwarddW's
+  // result by the fp32 summation order (one bf16 rounding step at most).
+  const bool tile = j.dprojw && j.tiles && tile_dxdw_ok(R, C);
+  if (!j.dprojw) TRY(op_proj_dw(c, b->attn_out, b->dOut, b->dProjw, R, C, partial, false));
   // projBackwarddX and computeD: one launch where the tiles of dAttn are whole heads
   float *dgamma = block ? b->ln_dgamma : nullptr, *dbeta = block ? b->ln_dbeta : nullptr;
-  if (tile_rows_ok(R, C, 1) && p->D == 64) {
+  if (j.d) {
     mla::TileRows t{b->dOut, {b->proj_w}, {b->dAttn}, 1, R, C};
     t.O = b->attn_out;
     t.Dv = b->Dsum;
@@ -664,8 +700,8 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
     TRY(flashAttentionBackwardWorkspace(b->dAttn, b->Dsum, b->l, b->q, b->k, b->v, b->dQ, b->dK, b->dV, attn_ws,
                                         attn_ws_bytes, p, s));
   }
-  uint16_t* lo = nullptr;  // no split when both hand-written kernels take the shape
-  if (!tile && std::max(split_need(R, C, true, true), split_need(R, C, false, true))) {
+  uint16_t* lo = nullptr;  // no split when hand-written kernels take both products
+  if (!j.dprojw && std::max(split_need(R, C, true, j.tiles), split_need(R, C, false, j.tiles))) {
     TRY(split_dq(c, b->dQ, e, split));  // one split serves both consumers
     lo = split + e;
   } else {
@@ -674,7 +710,7 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
   if (tile) {
     TRY(tile_grad(c, mla::TileGrad{b->dX, b->dQ, {b->q_w, b->k_w, b->v_w}, {b->X, b->X, b->X, b->attn_out},
                                    {nullptr, b->dK, b->dV, b->dOut}, {b->dQw, b->dKw, b->dVw, b->dProjw}, 0, 4, R, C}, partial, false));
-  } else if (fuse_pdw) {
+  } else if (j.dprojw) {
     // computeGradDx and the four weight gradients in one launch (dX tiles first, then the
     // weight-gradient items, which start as the dX tiles finish), then the reduction
     if (!c.query && mla::launch_grad_dxdw4(b->dX, b->X, b->dQ, b->dK, b->dV, b->q_w, b->k_w, b->v_w, b->attn_out,
@@ -682,8 +718,8 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
                                            c.stream) != hipSuccess)
       return METALLLM_ATTN_E_LAUNCH;
   } else {
-    TRY(op_grad_dx(c, b->dX, b->q_w, b->k_w, b->v_w, b->dQ, split, lo, b->dK, b->dV, R, C, true, false));
-    TRY(op_grad_dw(c, b->X, b->dQ, split, lo, b->dK, b->dV, b->dQw, b->dKw, b->dVw, R, C, partial, true, false));
+    TRY(op_grad_dx(c, b->dX, b->q_w, b->k_w, b->v_w, b->dQ, split, lo, b->dK, b->dV, R, C, j.tiles, false));
+    TRY(op_grad_dw(c, b->X, b->dQ, split, lo, b->dK, b->dV, b->dQw, b->dKw, b->dVw, R, C, partial, j.tiles, false));
   }
   if (c.query) return METALLLM_ATTN_OK;
   if (block)  // model.h:692-695: cast of dX, ln1 backward and the skip add
@@ -695,6 +731,14 @@ int encode(const Ctx& c, int phase, const metalllmSublayerBuffers* b, const Atte
   return METALLLM_ATTN_OK;
 }
 
+// bf16 elements of the dQ split and floats of weight-gradient partials that phase 1 may use.
+void phase_scratch(const metalllmSublayerBuffers* b, const AttentionParams* p, size_t& split, size_t& partial) {
+  const int R = (int)(p->B * p->M), C = (int)p->N;
+  const Joins j = joins(1, b, p);
+  split = j.dprojw ? 0 : std::max(split_need(R, C, true, j.tiles), split_need(R, C, false, j.tiles));
+  partial = partial_need(R, C, j.tiles && (j.dprojw || proj_dw_apart(b->attn_out, b->dOut, b->dProjw, R, C)));
+}
+
 int build_graph(metalllmSublayerGraph* g, const metalllmSublayerBuffers* b, const AttentionParams* p) {
   const int R = (int)(p->B * p->M), C = (int)p->N;
   if (rocblas_create_handle(&g->h) != rocblas_status_success) {
@@ -702,9 +746,9 @@ int build_graph(metalllmSublayerGraph* g, const metalllmSublayerBuffers* b, cons
     return METALLLM_ATTN_E_LIBRARY;
   }
   if (g->phase == 1) {
-    const size_t split = std::max(split_need(R, C, true, true), split_need(R, C, false, true));
+    size_t split = 0, partial = 0;
+    phase_scratch(b, p, split, partial);
     if (split && hipMalloc((void**)&g->split, split * sizeof(uint16_t)) != hipSuccess) g->split = nullptr;
-    const size_t partial = partial_need(R, C, true);
     if (partial && hipMalloc((void**)&g->partial, partial * sizeof(float)) != hipSuccess) g->partial = nullptr;
     TRY(metalllmAttnBackwardWorkspaceSize(p, &g->attn_ws_bytes));
     if (hipMalloc(&g->attn_ws, g->attn_ws_bytes) != hipSuccess) g->attn_ws = nullptr;
@@ -753,13 +797,20 @@ int metalllmSublayerEncode(int phase, const metalllmSublayerBuffers* b, const At
   TRY(u.s.rc);
   uint64_t ws = 0;
   if (phase == 1) {
-    TRY(ensure(u.s.st->split, u.s.st->split_elems, std::max(split_need(R, C, true, true), split_need(R, C, false, true)),
-               u.c.stream));
-    TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial_need(R, C, true), u.c.stream));
+    size_t split = 0, partial = 0;
+    phase_scratch(b, p, split, partial);
+    TRY(ensure(u.s.st->split, u.s.st->split_elems, split, u.c.stream));
+    TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial, u.c.stream));
     TRY(metalllmAttnBackwardWorkspaceSize(p, &ws));
     TRY(ensure(u.s.st->attn_ws, u.s.st->attn_ws_bytes, (size_t)ws, u.c.stream));
   }
   return encode(u.c, phase, b, p, u.s.st->split, u.s.st->partial, u.s.st->attn_ws, ws);
+}
+
+int metalllmSublayerRoute(int phase, const metalllmSublayerBuffers* b, const AttentionParams* p) {
+  TRY(check_phase(phase, b, p));
+  const Joins j = joins(phase, b, p);
+  return phase == 0 ? (j.residual ? 1 : 0) : (j.d ? 1 : 0) | (j.dprojw ? 2 : 0) | (j.tiles ? 4 : 0);
 }
 
 int metalllmSublayerReserve(const AttentionParams* p) {

@@ -39,7 +39,8 @@ def _L():
         L.metalllmSublayerGraphLaunch.argtypes = [vp, vp]
         L.metalllmSublayerGraphDestroy.argtypes = [vp]
         L.metalllmSublayerReserve.argtypes = [pp]
-        for f in (L.metalllmSublayerReserve, L.computeQKV, L.projForward, L.projBackwarddW, L.projBackwarddX, L.computeGradDx, L.computeGradDw,
+        L.metalllmSublayerRoute.argtypes = [ctypes.c_int, bp, pp]
+        for f in (L.metalllmSublayerRoute, L.metalllmSublayerReserve, L.computeQKV, L.projForward, L.projBackwarddW, L.projBackwarddX, L.computeGradDx, L.computeGradDw,
                   L.metalllmSublayerEncode, L.metalllmSublayerGraphCreate,
                   L.metalllmSublayerGraphLaunch, L.metalllmSublayerGraphDestroy):
             f.restype = ctypes.c_int
@@ -110,6 +111,13 @@ def encode_phase(phase: int, bufs: SublayerBuffers, p: AttentionParams, stream=N
     """metalllmSublayerEncode: enqueue phase 0 (forward) or 1 (backward) eagerly."""
     _check(_L().metalllmSublayerEncode(phase, ctypes.byref(bufs), ctypes.byref(p), _stream(stream)),
            "metalllmSublayerEncode")
+
+
+def route(phase: int, bufs: SublayerBuffers, p: AttentionParams) -> int:
+    """metalllmSublayerRoute (test hook): which dispatches a phase joins in one launch, as bits."""
+    r = _L().metalllmSublayerRoute(phase, ctypes.byref(bufs), ctypes.byref(p))
+    _check(min(r, 0), "metalllmSublayerRoute")
+    return r
 
 
 class PhaseGraph:

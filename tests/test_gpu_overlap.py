@@ -78,3 +78,66 @@ def test_products(gpu, S, R, H):
     for name, t, r in zip("qkv", (q, k, v), O.computeQKV(X, *Ws, threads=16)):
         bad, mx = bf_err(to_np(t), r)
         assert bad == 0, (name, mx)
+
+
+# (buffer, buffers whose memory it takes, in a row): each allowed by the order of the phase's calls
+REUSE = [("dK", ["attn_out"]), ("dV", ["attn_out"]), ("dK", ["dOut"]), ("dQ", ["attn_out", "dOut"]), ("dX", ["dOut", "attn_out"]),
+         ("Dsum", ["dOut"]), ("dKw", ["q_w"]), ("dX", ["q", "k"]), ("dX_bf16", ["dAttn"]), ("dX", ["dQ"])]
+
+
+@pytest.mark.parametrize("B,T,H", [(3, 320, 5), (2, 256, 6), (1, 64, 1)])
+def test_encoder_backward(gpu, S, B, T, H):
+    """Phase 1, eager and as a graph, with an output in the memory of buffers that no later call of the
+    phase reads, against the same phase on separate buffers. (dX over dQ is read later, by
+    computeGradDw: only where the library path runs, from its split of dQ.)"""
+    import torch
+    C = 64 * H
+    rng = np.random.default_rng(B * T + C)
+    g = lambda shape, sc=1.0: to_gpu(bf(rng, shape, sc), gpu)
+    sub = S.Sublayer(g((B, T, C)), *[g((C, C), 0.05) for _ in range(4)], H=H)
+    sub.dOut.copy_(g((B, T, C)))
+    sub.encode(0)
+    sub.encode(1)
+    torch.cuda.synchronize()
+    names = dict(dAttn="dO", Dsum="Dv", dQ="dQ", dK="dK", dV="dV", dX="dX", dQw="dWq", dKw="dWk", dVw="dWv", dProjw="dWp",
+                 dX_bf16="dXb", attn_out="o", dOut="dOut", q="q", k="k", q_w="Wq")
+    keep = {n: getattr(sub, a).clone() for n, a in names.items()}
+    for out, into in REUSE:
+        if (out, into) == ("dX", ["dQ"]) and C % 128 == 0:
+            continue
+        print(f"case B={B} T={T} C={C} {out} in {'+'.join(into)}", flush=True)
+        inputs = {n: keep[n] for n in ("attn_out", "dOut", "q", "k", "q_w")}
+        mem = torch.empty(max(sum(keep[n].nbytes for n in into), keep[out].nbytes), dtype=torch.uint8, device=gpu)
+        views, at = {}, 0
+        for n in into:
+            views[n] = mem[at:at + keep[n].nbytes].view(keep[n].dtype).view(keep[n].shape)
+            at += keep[n].nbytes
+        views[out] = mem[:keep[out].nbytes].view(keep[out].dtype).view(keep[out].shape)
+        b = sub.buffers()
+        for n, v in views.items():
+            setattr(b, n, v.data_ptr())
+
+        def check(run, what):
+            for n, a in names.items():
+                if n not in inputs:
+                    getattr(sub, a).fill_(float("nan"))
+            for n, v in inputs.items():
+                (views[n] if n in views else getattr(sub, names[n])).copy_(v)
+            run()
+            torch.cuda.synchronize()
+            for n, a in names.items():
+                if n in inputs or n in into:
+                    continue
+                got, ref = to_np(views.get(n, getattr(sub, a))), to_np(keep[n])
+                if got.dtype == np.float32:
+                    assert f32_err(got, ref) <= (1e-4 if n == "dQw" else 1e-5), (what, n)
+                else:
+                    assert bf_err(got, ref)[0] == 0, (what, n)
+
+        check(lambda: S.encode_phase(1, b, sub.p), "eager")
+        graph = S.PhaseGraph(1, b, sub.p)
+        for _ in range(2):
+            check(graph.launch, "graph")
+        graph.close()
+        for n, v in inputs.items():
+            getattr(sub, names[n]).copy_(v)
