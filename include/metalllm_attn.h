@@ -116,6 +116,10 @@ int metalllmAttnBackwardWorkspaceSize(const AttentionParams* p, uint64_t* bytes)
  * it runs flashAttentionBackward's kernel writing dQ instead of adding into it (there the
  * recomputation in one launch is faster than the dS round trip's two), so dQ, dK and dV equal
  * flashAttentionBackward's into a zeroed dQ bit for bit.
+ * An output may lie in an input's memory where the kernels allow it: dV in v's, and dQ in that of
+ * q, v and dZ, at D = 128; dV in v's and dK in k's at D = 64 with M <= 256 (there in
+ * flashAttentionBackward too). Such a call runs the
+ * stored-dS kernels or the fused one at any number of pairs.
  * No counterpart in the reference. */
 int flashAttentionBackwardWorkspace(const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
                                     const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
@@ -339,6 +343,15 @@ int metalllmSublayerRoute(int phase, const metalllmSublayerBuffers* b, const Att
 /* Static description of an error code (no counterpart in the reference, which has no error
  * path per kernel; model.h:333-336,361-365 only print). */
 const char* metalllmAttnErrorString(int code);
+
+/* Test hook (no counterpart in the reference): the kernels that flashAttentionBackward (workspace = 0)
+ * or flashAttentionBackwardWorkspace (1) runs for this shape and these buffers: 0 = the fused
+ * short-sequence kernel, 1 = dK/dV and dQ in one launch, 2 = dK/dV, then dQ recomputing the softmax,
+ * 3 = dK/dV storing dS, then dQ from it; or a negative error code for a bad shape. Host-only:
+ * nothing is read through the pointers. */
+int metalllmAttnBackwardRoute(int workspace, const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
+                              const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
+                              const AttentionParams* p);
 
 /* Test hook (no counterpart in the reference): writes, for workgroup ids 0..count-1 of the
  * forward (kind 0), backward dK/dV (kind 1) or backward dQ (kind 2) grid of shape p, the

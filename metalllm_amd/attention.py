@@ -31,7 +31,7 @@ EXPORTED = ("flashAttentionForward", "computeD", "flashAttentionBackward", "meta
             "layernormForward", "layernormBackward",
             "metalllmSublayerGraphCreate", "metalllmSublayerGraphLaunch", "metalllmSublayerGraphDestroy",
             "metalllmSublayerReserve", "flashAttentionBackwardNoAlloc", "metalllmAttnForwardItems",
-            "metalllmSublayerRoute")
+            "metalllmSublayerRoute", "metalllmAttnBackwardRoute")
 NOALLOC_SCRATCH_BYTES = 64 << 20  # METALLLM_ATTN_NOALLOC_SCRATCH_BYTES
 
 
@@ -78,6 +78,8 @@ def _lib():
         L.metalllmAttnErrorString.restype = ctypes.c_char_p
         L.metalllmAttnWorkMap.argtypes = [ctypes.c_int, pp, ctypes.c_void_p, ctypes.c_int32]
         L.metalllmAttnWorkMap.restype = ctypes.c_int
+        L.metalllmAttnBackwardRoute.argtypes = [ctypes.c_int] + [vp] * 9 + [pp]
+        L.metalllmAttnBackwardRoute.restype = ctypes.c_int
         L.metalllmAttnForwardItems.argtypes = [pp, ctypes.c_int32, ctypes.c_void_p, ctypes.c_int32]
         L.metalllmAttnForwardItems.restype = ctypes.c_int
         _LIB = L
@@ -185,6 +187,22 @@ def backward_part(part: int, dZ, d, l, q, k, v, dQ, dK, dV, stream=None, params:
     _check(_lib().metalllmAttnBackwardPart(part, _ptr(dZ), _ptr(d), _ptr(l), _ptr(q), _ptr(k), _ptr(v), _ptr(dQ),
                                            _ptr(dK), _ptr(dV), wp, wn, ctypes.byref(p), _stream(stream)),
            "metalllmAttnBackwardPart")
+
+
+# backward_route: the kernels of a backward call
+FUSED, JOINT, TWO, STORED = range(4)
+
+
+def backward_route(B: int, T: int, H: int, D: int, workspace: bool, addresses=None) -> int:
+    """metalllmAttnBackwardRoute (test hook): the kernels that flashAttentionBackward, or with
+    `workspace` flashAttentionBackwardWorkspace, runs. addresses: of dZ, d, l, q, k, v, dQ, dK and dV
+    (none: buffers apart from each other)."""
+    p = AttentionParams.of(B, T, H, D)
+    if addresses is None:
+        addresses = [(1 << 40) * (i + 1) for i in range(9)]
+    r = _lib().metalllmAttnBackwardRoute(int(workspace), *addresses, ctypes.byref(p))
+    _check(min(r, 0), "metalllmAttnBackwardRoute")
+    return r
 
 
 def attention_forward(q, k, v, stream=None):

@@ -5,6 +5,7 @@
 
 #include "../../include/metalllm_attn.h"
 #include "attn_launch.hpp"
+#include "overlap.hpp"
 
 namespace {
 
@@ -20,6 +21,26 @@ int validate(const AttentionParams* p) {
 bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 
 float head_scale(uint32_t D) { return 1.0f / std::sqrt((float)D); }  // attention.metal:109,268
+
+// Kernels of a backward entry point (metalllmAttnBackwardRoute's values).
+enum Route { kFused = 0, kJoint = 1, kTwo = 2, kStored = 3 };
+
+// acc: flashAttentionBackward, else flashAttentionBackwardWorkspace. An output may lie in the memory of
+// an input that the kernels after the one writing it do not read, where that one reads an element
+// only in the workgroup that replaces it: dV in v's (and in the fused kernel, which keeps a pair's K in
+// LDS, dK in k's); dQ, written from the stored dS and k alone, in those of q, v and dZ. In the joint
+// launch dQ's workgroups may read any input after dK's and dV's have ended, so it takes outputs apart
+// from the inputs only. The kernels for the others follow from D and T alone, so that a caller can
+// plan for them.
+Route backward_route(const mla::BwdArgs& a, int D, bool acc) {
+  const size_t e = (size_t)a.B * a.T * a.H * D, stat = (size_t)a.B * a.H * a.T;
+  const bool apart = !mla::any_overlap({{a.dQ, 4 * e}, {a.dK, 2 * e}, {a.dV, 2 * e}},
+                                       {{a.dO, 2 * e}, {a.Dv, 4 * stat}, {a.lse, 4 * stat}, {a.q, 2 * e}, {a.k, 2 * e}, {a.v, 2 * e}});
+  const int pairs = a.B * a.H;
+  if (!apart) return D == 64 && a.T <= 256 ? kFused : (acc || D == 64) ? kTwo : kStored;
+  if (mla::backward_is_short(a.T, D, pairs)) return kFused;
+  return acc || mla::workspace_recomputes(a.T, D, pairs) ? kJoint : kStored;
+}
 
 // One part of a backward entry point (metalllmAttnBackwardPart), or with `whole` the entry point
 // whose first part it is (0: flashAttentionBackward, 2: flashAttentionBackwardWorkspace).
@@ -44,18 +65,25 @@ int backward(int part, const uint16_t* dZ, const float* d, const float* l, const
   }
   const bool first = part == 0 || part == 2;
   hipError_t e = hipSuccess;
-  if (mla::backward_is_short(a.T, D, a.B * a.H)) {
-    // one fused kernel computes dK, dV and dQ; the second part has nothing left to do
-    if (first) e = mla::launch_backward_short(a, acc, s);
-  } else if (acc || mla::workspace_recomputes(a.T, D, a.B * a.H)) {
-    e = whole   ? mla::launch_backward_both(a, D, acc, s)
-        : first ? mla::launch_backward(a, D, s)
-                : mla::launch_backward_dq(a, D, acc, s);
-  } else {
-    // dK/dV storing dS into the workspace, then dQ = dS.K
-    a.dS = (uint16_t*)workspace;
-    if (first) e = mla::launch_backward(a, D, s);
-    if (e == hipSuccess && (whole || !first)) e = mla::launch_backward_dqs(a, D, s);
+  switch (backward_route(a, D, acc)) {
+    case kFused:  // one kernel computes dK, dV and dQ; the second part has nothing left to do
+      if (first) e = mla::launch_backward_short(a, acc, s);
+      break;
+    case kJoint:
+      if (whole) {
+        e = mla::launch_backward_both(a, D, acc, s);
+        break;
+      }
+      [[fallthrough]];
+    case kTwo:  // dK/dV, then dQ
+      if (first) e = mla::launch_backward(a, D, s);
+      if (e == hipSuccess && (whole || !first)) e = mla::launch_backward_dq(a, D, acc, s);
+      break;
+    case kStored:  // dK/dV storing dS into the workspace, then dQ = dS.K
+      a.dS = (uint16_t*)workspace;
+      if (first) e = mla::launch_backward(a, D, s);
+      if (e == hipSuccess && (whole || !first)) e = mla::launch_backward_dqs(a, D, s);
+      break;
   }
   return e == hipSuccess ? METALLLM_ATTN_OK : METALLLM_ATTN_E_LAUNCH;
 }
@@ -112,6 +140,15 @@ int flashAttentionBackwardWorkspace(const uint16_t* dZ, const float* d, const fl
                                     void* workspace, uint64_t workspace_bytes, const AttentionParams* p,
                                     metalllm_stream_t stream) {
   return backward(2, dZ, d, l, q, k, v, dQ, dK, dV, workspace, workspace_bytes, p, stream, true);
+}
+
+int metalllmAttnBackwardRoute(int workspace, const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
+                              const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
+                              const AttentionParams* p) {
+  const int rc = validate(p);
+  if (rc) return rc;
+  const mla::BwdArgs a{dZ, d, l, q, k, v, dQ, dK, dV, (int)p->M, (int)p->NH, (int)p->B, 0.0f};
+  return backward_route(a, (int)p->D, workspace == 0);
 }
 
 const char* metalllmAttnErrorString(int code) {

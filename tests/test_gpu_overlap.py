@@ -141,3 +141,41 @@ def test_encoder_backward(gpu, S, B, T, H):
         graph.close()
         for n, v in inputs.items():
             getattr(sub, names[n]).copy_(v)
+
+
+@pytest.mark.parametrize("B,T,H,D,into", [(2, 512, 4, 128, {"dV": "v"}), (1, 192, 3, 128, {"dQ": "q"}), (3, 576, 4, 128, {"dQ": "v", "dV": "v"}),
+                                          (1, 256, 6, 64, {"dV": "v", "dK": "k"}), (2, 128, 3, 64, {"dV": "v", "dK": "k"}),
+                                          (1, 192, 5, 64, {"dK": "k"})])
+def test_attention_backward(gpu, B, T, H, D, into):
+    """flashAttentionBackwardWorkspace with an output in the memory of an input (dQ, twice as long, also
+    in dZ's behind it; where dV is in v's as well, dQ in q's and dZ's) against separate buffers: dK and dV
+    bit for bit, dQ up to fp32 summation order. At D = 64 flashAttentionBackward as well."""
+    import torch
+    import metalllm_amd as M
+    from tests.attn_case import make_inputs
+    print(f"case B={B} T={T} H={H} D={D} {into}", flush=True)
+    q, k, v, g = (to_gpu(x, gpu) for x in make_inputs(B, T, H, D, 31))
+    out, lse = M.attention_forward(q, k, v)
+    Dv = torch.empty_like(lse)
+    M.computeD(g, out, Dv)
+    ws = torch.empty((M.workspace_bytes(B, T, H, D),), dtype=torch.uint8, device=gpu)
+    new = lambda: (torch.zeros((B, T, H, D), device=gpu), torch.empty_like(q), torch.empty_like(q))
+    ref = new()
+    M.flashAttentionBackwardWorkspace(g, Dv, lse, q, k, v, *ref, ws)
+    for entry in ("workspace", "add") if D == 64 else ("workspace",):
+        mem = torch.empty((4,) + q.shape, dtype=torch.bfloat16, device=gpu)  # q or v, dZ, then the others
+        first = "q" if into.get("dQ") != "v" or "dV" in into else "v"
+        i = dict(zip((first, "dZ", "v" if first == "q" else "q", "k"), mem.unbind(0)))
+        for n, t in (("q", q), ("k", k), ("v", v), ("dZ", g)):
+            i[n].copy_(t)
+        dQ, dK, dV = new()
+        if "dQ" in into:
+            dQ = mem[:2].view(torch.float32).view(q.shape)
+        dK, dV = i["k"] if "dK" in into else dK, i["v"] if "dV" in into else dV
+        if entry == "workspace":
+            M.flashAttentionBackwardWorkspace(i["dZ"], Dv, lse, i["q"], i["k"], i["v"], dQ, dK, dV, ws)
+        else:
+            M.flashAttentionBackward(i["dZ"], Dv, lse, i["q"], i["k"], i["v"], dQ, dK, dV)
+        torch.cuda.synchronize()
+        assert torch.equal(dK, ref[1]) and torch.equal(dV, ref[2])
+        assert (dQ - ref[0]).abs().max().item() <= 1e-5 * ref[0].abs().max().item()
