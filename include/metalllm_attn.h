@@ -163,7 +163,10 @@ int flashAttentionBackwardNoAlloc(const uint16_t* dZ, const float* d, const floa
 
 /* Sizes the current device's sublayer scratch (dQ split, weight-gradient partials, the phase
  * encoder's attention workspace) for shape p, synchronising the device if a buffer grows; the
- * GEMM entry points and metalllmSublayerEncode at shapes up to p then run without allocating.
+ * GEMM entry points at no more rows (B*M) and features than p's, and metalllmSublayerEncode with no
+ * larger B, M, NH and N, then run without allocating, whichever kernels the smaller shape takes: 4
+ * bytes per element of an activation and at most 128 per element of a weight, beside the workspace.
+ * (Where the device has no room for that, what p itself needs.)
  * No counterpart in the reference (model.h allocates every buffer once, :236-277). */
 int metalllmSublayerReserve(const AttentionParams* p);
 
@@ -339,6 +342,11 @@ int metalllmAttnBackwardPart(int part, const uint16_t* dZ, const float* d, const
  * products' buffers are apart, as their kernels on 64 x 64 tiles need. Negative error codes as
  * metalllmSublayerEncode. Host-only: nothing is read through the pointers. */
 int metalllmSublayerRoute(int phase, const metalllmSublayerBuffers* b, const AttentionParams* p);
+
+/* Test hook (no counterpart in the reference): the scratch that a call at shape p needs at most (bf16
+ * elements of the dQ split, floats of weight-gradient partials), and what metalllmSublayerReserve
+ * sizes for p. Host-only. */
+int metalllmSublayerScratch(const AttentionParams* p, uint64_t need[2], uint64_t reserved[2]);
 
 /* Static description of an error code (no counterpart in the reference, which has no error
  * path per kernel; model.h:333-336,361-365 only print). */

@@ -31,7 +31,7 @@ EXPORTED = ("flashAttentionForward", "computeD", "flashAttentionBackward", "meta
             "layernormForward", "layernormBackward",
             "metalllmSublayerGraphCreate", "metalllmSublayerGraphLaunch", "metalllmSublayerGraphDestroy",
             "metalllmSublayerReserve", "flashAttentionBackwardNoAlloc", "metalllmAttnForwardItems",
-            "metalllmSublayerRoute", "metalllmAttnBackwardRoute")
+            "metalllmSublayerRoute", "metalllmAttnBackwardRoute", "metalllmSublayerScratch")
 NOALLOC_SCRATCH_BYTES = 64 << 20  # METALLLM_ATTN_NOALLOC_SCRATCH_BYTES
 
 

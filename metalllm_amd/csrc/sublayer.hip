@@ -311,6 +311,44 @@ size_t partial_need(int R, int C, bool tiles) {
   return std::max(tile, 2 * (size_t)row_chunks(R) * C * C);
 }
 
+// For any buffers, apart or not (partial_need without tiles covers both).
+size_t any_split_need(int R, int C) { return std::max(split_need(R, C, true, false), split_need(R, C, false, false)); }
+
+// The most that a call of at most R rows and C features can need of either buffer, whichever kernels
+// it runs: a smaller shape may take the 64-wide tiles, whose row chunks grow as C shrinks, the 128-wide
+// ones, or the library, where a larger one does not.
+size_t split_bound(int R, int C) { return 2 * (size_t)R * C; }
+size_t partial_bound(int R, int C) {
+  int parts = 1;  // row_chunks of some row count up to R
+  while (parts < 16 && R >= 512 * 2 * parts) parts *= 2;
+  size_t n = 2 * (size_t)parts * C * C;
+  for (int c = 64; c <= C; c += 64) {
+    n = std::max({n, mla::tile_grad_partial_bound(R, c, 3, 4, false), mla::tile_grad_partial_bound(R, c, 0, 3, false),
+                  mla::tile_grad_partial_bound(R, c, 0, 4, true)});
+    if (c % 128 == 0)  // chunks follow the rows up to a limit
+      n = std::max({n, mla::grad_dw_one_partial_floats(R, c), mla::grad_dw_partial_floats(R, c), mla::grad_dw4_partial_floats(R, c)});
+  }
+  return n;
+}
+
+// Grows a buffer to `most`, or, where the device has no room for that, to `need`.
+template <typename T>
+int reserve(T*& buf, size_t& have, size_t most, size_t need) {
+  if (have >= most) return METALLLM_ATTN_OK;
+  T* grown = nullptr;
+  if (hipMalloc((void**)&grown, most * sizeof(T)) != hipSuccess) {
+    (void)hipGetLastError();  // not the next launch's error
+    return ensure(buf, have, need, nullptr);
+  }
+  if (buf && (hipDeviceSynchronize() != hipSuccess || hipFree(buf) != hipSuccess)) {
+    (void)hipFree(grown);
+    return METALLLM_ATTN_E_LIBRARY;
+  }
+  buf = grown;
+  have = most;
+  return METALLLM_ATTN_OK;
+}
+
 int xt_g_partials(const Ctx& c, const uint16_t* X, const uint16_t* G, int R, int C, int parts, float* out) {
   const float alpha = 1.0f, beta = 0.0f;
   const int Rs = R / parts;
@@ -813,6 +851,17 @@ int metalllmSublayerRoute(int phase, const metalllmSublayerBuffers* b, const Att
   return phase == 0 ? (j.residual ? 1 : 0) : (j.d ? 1 : 0) | (j.dprojw ? 2 : 0) | (j.tiles ? 4 : 0);
 }
 
+int metalllmSublayerScratch(const AttentionParams* p, uint64_t need[2], uint64_t reserved[2]) {
+  TRY(validate_gemm(p));
+  if (!need || !reserved) return METALLLM_ATTN_E_NULL;
+  const int R = (int)(p->B * p->M), C = (int)p->N;
+  need[0] = any_split_need(R, C);
+  need[1] = partial_need(R, C, false);
+  reserved[0] = split_bound(R, C);
+  reserved[1] = partial_bound(R, C);
+  return METALLLM_ATTN_OK;
+}
+
 int metalllmSublayerReserve(const AttentionParams* p) {
   TRY(validate_gemm(p));
   if (p->D != 64 && p->D != 128) return METALLLM_ATTN_E_HEADDIM;
@@ -822,11 +871,8 @@ int metalllmSublayerReserve(const AttentionParams* p) {
   TRY(metalllmAttnBackwardWorkspaceSize(p, &ws));
   Public u(nullptr);
   TRY(u.s.rc);
-  // what the library path of this shape would take too: a smaller shape may run it
-  const bool lib = !mla::grad_dw_fused_ok(R, C);
-  const size_t partial = std::max(partial_need(R, C, true), lib ? 2 * (size_t)row_chunks(R) * C * C : 0);
-  TRY(ensure(u.s.st->split, u.s.st->split_elems, lib ? 2 * (size_t)R * C : 0, nullptr));
-  TRY(ensure(u.s.st->partial, u.s.st->partial_elems, partial, nullptr));
+  TRY(reserve(u.s.st->split, u.s.st->split_elems, split_bound(R, C), any_split_need(R, C)));
+  TRY(reserve(u.s.st->partial, u.s.st->partial_elems, partial_bound(R, C), partial_need(R, C, false)));
   TRY(ensure(u.s.st->attn_ws, u.s.st->attn_ws_bytes, (size_t)ws, nullptr));
   return METALLLM_ATTN_OK;
 }

@@ -526,23 +526,31 @@ struct Chunks {
 
 // Row chunks of the weight gradients: as many as bring a wave's chain of units (R / 64 / 4 for a
 // bf16 weight, twice that for dQw) down to about half of what every wave of the chip has to do, when
-// the undivided chain is longer than all of it.
-Chunks grad_chunks(int R, int C, int w0, int w1, bool dx) {
+// the undivided chain is longer than all of it (which `divide` takes for granted: the number of chunks
+// then only grows with R).
+Chunks grad_chunks(int R, int C, int w0, int w1, bool dx, bool divide = false) {
   if (w1 <= w0) return {1, 1};
   const double tiles = (double)(C / 64) * (C / 64), rows = R / 64.0;
   const double mean = tiles * rows * ((dx ? 4 : 0) + (w1 - w0) + (w0 == 0 ? 1 : 0)) / (256 * 8);
   const double chain = rows / 4 * (w0 == 0 ? 2 : 1);
-  if (chain <= 1.25 * mean + 8) return {1, 1};
+  if (!divide && chain <= 1.25 * mean + 8) return {1, 1};
   const int n = (int)(rows / 4 / std::max(4.0, mean / 2) + 0.999);
   return {w0 == 0 ? std::max(1, 2 * n) : 0, std::max(1, n)};
+}
+
+size_t partial_floats(const Chunks& k, int C, int w0, int w1) {
+  if (k.nkv == 1 && k.nq <= 1) return 0;
+  return (size_t)(k.nq + (w1 - std::max(w0, 1)) * k.nkv) * C * C;
 }
 
 }  // namespace
 
 size_t tile_grad_partial_floats(int R, int C, int w0, int w1, bool dx) {
-  const Chunks k = grad_chunks(R, C, w0, w1, dx);
-  if (k.nkv == 1 && k.nq <= 1) return 0;
-  return (size_t)(k.nq + (w1 - std::max(w0, 1)) * k.nkv) * C * C;
+  return partial_floats(grad_chunks(R, C, w0, w1, dx), C, w0, w1);
+}
+
+size_t tile_grad_partial_bound(int R, int C, int w0, int w1, bool dx) {
+  return partial_floats(grad_chunks(R, C, w0, w1, dx, true), C, w0, w1);
 }
 
 hipError_t launch_tile_grad(TileGrad a, float* partial, bool accumulate, hipStream_t s) {

@@ -41,6 +41,8 @@ struct TileGrad {
 };
 // Floats of `partial` that launch_tile_grad needs for these products (0: none).
 size_t tile_grad_partial_floats(int R, int C, int w0, int w1, bool dx);
+// The most it needs for any multiple of 64 rows up to R.
+size_t tile_grad_partial_bound(int R, int C, int w0, int w1, bool dx);
 hipError_t launch_tile_grad(TileGrad a, float* partial, bool accumulate, hipStream_t s);
 
 }  // namespace mla

@@ -40,7 +40,8 @@ def _L():
         L.metalllmSublayerGraphDestroy.argtypes = [vp]
         L.metalllmSublayerReserve.argtypes = [pp]
         L.metalllmSublayerRoute.argtypes = [ctypes.c_int, bp, pp]
-        for f in (L.metalllmSublayerRoute, L.metalllmSublayerReserve, L.computeQKV, L.projForward, L.projBackwarddW, L.projBackwarddX, L.computeGradDx, L.computeGradDw,
+        L.metalllmSublayerScratch.argtypes = [pp, ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint64)]
+        for f in (L.metalllmSublayerRoute, L.metalllmSublayerScratch, L.metalllmSublayerReserve, L.computeQKV, L.projForward, L.projBackwarddW, L.projBackwarddX, L.computeGradDx, L.computeGradDw,
                   L.metalllmSublayerEncode, L.metalllmSublayerGraphCreate,
                   L.metalllmSublayerGraphLaunch, L.metalllmSublayerGraphDestroy):
             f.restype = ctypes.c_int
@@ -118,6 +119,14 @@ def route(phase: int, bufs: SublayerBuffers, p: AttentionParams) -> int:
     r = _L().metalllmSublayerRoute(phase, ctypes.byref(bufs), ctypes.byref(p))
     _check(min(r, 0), "metalllmSublayerRoute")
     return r
+
+
+def scratch(p: AttentionParams):
+    """metalllmSublayerScratch (test hook): (split elements, partial floats) that a call at p needs at
+    most, and the two that reserve(p) sizes."""
+    need, reserved = (ctypes.c_uint64 * 2)(), (ctypes.c_uint64 * 2)()
+    _check(_L().metalllmSublayerScratch(ctypes.byref(p), need, reserved), "metalllmSublayerScratch")
+    return tuple(need), tuple(reserved)
 
 
 class PhaseGraph:
