@@ -203,25 +203,66 @@ int split_dq(const Ctx& c, const float* dQ, size_t elems, uint16_t* split) {
 
 // Whether the 64 x 64 tile kernels (sublayer_tile.hip) take a product: up to large sizes where the
 // 128-wide kernels (sublayer_gemm.hip) and the library's large tiles do not fit, else small ones, which
-// they run in fewer and shorter dependent steps. A library call also costs about 21 us of host time,
-// these launches about 3. Device times, tile kernel against library or 128-wide kernel:
-//   rows, by units of 64 x 64 x 64: C = 768 computeQKV R = 1024 13 / 12 us, 2048 (13824 units) 19 / 17,
-//     4096 32 / 26; projForward 4096 12.0 / 14.6, 6144 (13824) 17 / 14; C = 384 computeQKV 8192 (13824)
-//     22 / 22, projForward 16384 (9216) 15.7 / 14.1; C = 448 computeQKV 8192 27 / 36, 16384 48 / 62
-//   computeGradDx, the dX + dW launch: C = 768 R = 2048 22 / 51, 6144 52 / 54, 8192 64 / 57 (with the
-//     weights break-even at 3072); C = 384 12288 32 / 32, 16384 38 / 35; C = 448 16384 49 / 92
-//   computeGradDw: C = 768 R = 2048 27 / 32, 4096 44 / 41; C = 384 16384 41 / 51; C = 448 16384 55 / 111
-//   projBackwarddW: C = 768 R = 4096 21 / 24, 8192 28 / 28, 16384 41 / 38; C = 384 16384 21 / 24
-bool tile_rows_ok(int R, int C, int n) {
-  return C % 64 == 0 && (int64_t)((R + 63) / 64) * (C / 64) * (C / 64) * n <= (C % 128 ? 64000 : 14000);
+// they run in fewer and shorter dependent steps. Device times in us, tile kernel against library or
+// 128-wide kernel, launches queued ahead of the host.
+//
+// Row products, by units of 64 x 64 x 64. A library call also costs 16-21 us of host time, these
+// launches about 3, which a program that calls one after another pays: the lines for C in multiples of
+// 128 lie where the device loses 1-2 us at most and such a program still gains (C = 768, eager:
+// projForward R = 4096 11.4 / 16.3; computeQKV R = 1024 11.7 / 16.5, but R = 2048 17.9 / 16.5).
+//   computeQKV, against the library's one batched call 7000 units: C = 768 R = 640 (4320) 8.1 / 9.4, 1024 (6912)
+//     12.0 / 10.9, 1536 (10368) 15.0 / 13.2, 2048 (13824) 19.1 / 16.0 (14000 against three calls, which take
+//     the time of three projections: 26); C = 384 R = 2432 (4104) 9.3 / 9.2,
+//     4096 (6912) 13.5 / 12.5; C = 1024 R = 512 (6144) 13.1 / 11.1, 1024 (12288) 20.2 / 14.6
+//   projForward, 10500 units and 1024 tiles (few features: short sums, the copies of x bound): C = 768 R =
+//     3840 (8640) 11.9 / 13.5, 4480 (10080) 13.9 / 12.4, 6144 (13824) 17.4 / 13.9; C = 256 R = 7936 (496
+//     tiles) 5.5 / 7.2, 16000 (1000) 9.2 / 8.6, 28032 (1752) 15.2 / 11.1. With the encoder's residual add,
+//     which saves a pass over the rows, a phase is level at 1152 tiles (C = 384 R = 12288, C = 512 R = 9216)
+//   projBackwarddX, 7000 units and 768 tiles: C = 768 R = 2432 (5472) 8.3 / 8.4, 3072 (6912) 11.3 / 9.5,
+//     4480 (10080) 13.8 / 11.0; C = 384 R = 3584 (336 tiles) 5.9 / 6.7, 7168 (672) 9.1 / 7.6. With computeD,
+//     the phase is level at 768 tiles (C = 768 R = 4096 123.1 / 124.4) and loses 4 us at 960
+//   other multiples of 64: computeQKV wins at 320-704 features nearly throughout (C = 448 6976 rows 23 /
+//     45, 27008 79 / 92), not far beyond 12000 units from 768 on (C = 960 R = 768 15.0 / 15.9, 1536 24.7 /
+//     19.9; C = 1216 R = 448 13.6 / 13.9, 960 24.9 / 19.2), nor 16000 below 256 (C = 192 R = 37952 36.9 /
+//     39.6, 56896 51 / 41). The projections: below 256 features 16000 units (C = 192 R = 113792 36.6 / 54,
+//     170688 52 / 39); from 768 on 20000 (C = 960 R = 4544 19.4 / 18.9, 12800 44 / 29; C = 1216 R = 4224 24.2 /
+//     26.1); between, alone within 10% either way on the mean of the sizes (C = 448 R = 58752 59 / 62, C =
+//     576 18944 32 / 21, 25280 39 / 46), and in the encoder, whose results are the entry points' bit for
+//     bit, ahead by the pass saved (16384 x 448, 4 bytes an element: about 8 us)
+// Gradient products:
+//   computeGradDx, the dX + dW launch: C = 768 R = 2048 23 / 52, 2944 34 / 52, 6144 52 / 54, 8192 64 / 57
+//     (with the weights break-even at 3072); C = 384 12160 33 / 34, 16384 38 / 35; C = 448 14912 46 / 92. With
+//     few features its tiles bound it, 1500 of them: C = 256 R = 23296 (1456) 30.3 / 30.2, 27392 (1712)
+//     35.0 / 31.7; C = 128 R = 32896 (1028) 19.0 / 19.7, 54912 (1716) 26.2 / 22.5
+//   computeGradDw: C = 768 R = 2944 32 / 36, 4096 44 / 41; C = 512 6784 32.9 / 33.0; up to 384 features,
+//     where 192 divides them, C = 384 24320 56 / 66, else C = 256 38400 42.7 / 43.1, 54912 54.5 / 52.1; C =
+//     448 R = 14912 48 / 125
+//   projBackwarddW: C = 768 R = 5632 23 / 25, 8064 28.6 / 28.0, 16384 41 / 38; C = 384 R = 27648 26 / 28, 32512
+//     31 / 29; C = 1024 R = 4480 21 / 28; C = 448 R = 29888 33 / 41
+enum Rows { kQkvBatched, kQkv, kProjForward, kProjBackward };
+bool tile_rows_ok(int R, int C, Rows what) {
+  if (C % 64) return false;
+  const int64_t tiles = (int64_t)((R + 63) / 64) * (C / 64) * (what <= kQkv ? 3 : 1), units = tiles * (C / 64);
+  const bool wide = C % 128 == 0;
+  switch (what) {
+    case kQkv: return units <= (wide ? 14000 : 64000);
+    case kQkvBatched: return units <= (wide ? 7000 : C < 256 ? 16000 : C < 768 ? 64000 : 12000);
+    case kProjForward:
+      if (wide) return units <= 10500 && tiles <= 1024;
+      break;
+    case kProjBackward:
+      if (wide) return units <= 7000 && tiles <= 768;
+  }
+  return units <= (C < 256 ? 16000 : C < 768 ? 64000 : 20000);
 }
 bool small_product(int R, int C, double limit) { return (double)R * C * C <= limit; }
 constexpr double kTileBeforeLibrary = 3e10;
 bool tile_dx_ok(int R, int C) {
-  return C % 64 == 0 && small_product(R, C, mla::grad_dx_fused_ok(R, C) ? 1.8e9 : kTileBeforeLibrary);
+  if (!mla::grad_dx_fused_ok(R, C)) return C % 64 == 0 && small_product(R, C, kTileBeforeLibrary);
+  return small_product(R, C, 1.8e9) && (int64_t)(R / 64) * (C / 64) <= 1500;
 }
 bool tile_dw_ok(int R, int C) {  // computeGradDw
-  const double limit = mla::grad_dw_fused_ok(R, C) ? (C <= 384 ? 3.6e9 : 1.8e9) : kTileBeforeLibrary;
+  const double limit = !mla::grad_dw_fused_ok(R, C) ? kTileBeforeLibrary : C > 384 ? 1.8e9 : C % 192 ? 2.6e9 : 3.6e9;
   return C % 64 == 0 && R % 64 == 0 && small_product(R, C, limit);
 }
 bool tile_dw_one_ok(int R, int C) {  // projBackwarddW
@@ -413,12 +454,13 @@ int op_qkv(const Ctx& c, const uint16_t* X, uint16_t* q, uint16_t* k, uint16_t* 
            const uint16_t* k_w, const uint16_t* v_w, int R, int C) {
   // distances in bf16 elements, from the integer addresses (the buffers may be separate allocations)
   const auto at = [](const uint16_t* ptr) { return (intptr_t)(uintptr_t)ptr; };
-  if (tile_rows_ok(R, C, 3) && qkv_apart(X, q, k, v, q_w, k_w, v_w, R, C))
-    return tile_rows(c, mla::TileRows{X, {q_w, k_w, v_w}, {q, k, v}, 3, R, C}, false);
   const intptr_t bw = at(k_w) - at(q_w), by = at(k) - at(q);
   const intptr_t dw = bw / 2, dy = by / 2;
-  if (bw % 2 == 0 && by % 2 == 0 && dw >= 0 && at(v_w) - at(k_w) == bw && dy >= (intptr_t)R * C &&
-      at(v) - at(k) == by) {
+  const bool batched = bw % 2 == 0 && by % 2 == 0 && dw >= 0 && at(v_w) - at(k_w) == bw && dy >= (intptr_t)R * C &&
+                       at(v) - at(k) == by;
+  if (tile_rows_ok(R, C, batched ? kQkvBatched : kQkv) && qkv_apart(X, q, k, v, q_w, k_w, v_w, R, C))
+    return tile_rows(c, mla::TileRows{X, {q_w, k_w, v_w}, {q, k, v}, 3, R, C}, false);
+  if (batched) {
     const float alpha = 1.0f, beta = 0.0f;
     // row-major Y_i = X . W_i; column-major Y_i^T = W_i^T . X^T
     const rocblas_status st = rocblas_gemm_strided_batched_ex(
@@ -433,7 +475,7 @@ int op_qkv(const Ctx& c, const uint16_t* X, uint16_t* q, uint16_t* k, uint16_t* 
 }
 
 int op_proj_fwd(const Ctx& c, const uint16_t* attn_out, const uint16_t* proj_w, uint16_t* out, int R, int C) {
-  if (tile_rows_ok(R, C, 1) && rows_apart(attn_out, proj_w, out, R, C))
+  if (tile_rows_ok(R, C, kProjForward) && rows_apart(attn_out, proj_w, out, R, C))
     return tile_rows(c, mla::TileRows{attn_out, {proj_w}, {out}, 1, R, C}, false);
   return gemm_rm(c, false, false, R, C, C, attn_out, BF, C, proj_w, BF, C, 0.0f, out, BF, C);
 }
@@ -460,7 +502,7 @@ int op_proj_dw(const Ctx& c, const uint16_t* attn_out, const uint16_t* dZ, uint1
 }
 
 int op_proj_dx(const Ctx& c, const uint16_t* dZ, const uint16_t* proj_w, uint16_t* dAttn, int R, int C) {
-  if (tile_rows_ok(R, C, 1) && rows_apart(dZ, proj_w, dAttn, R, C))
+  if (tile_rows_ok(R, C, kProjBackward) && rows_apart(dZ, proj_w, dAttn, R, C))
     return tile_rows(c, mla::TileRows{dZ, {proj_w}, {dAttn}, 1, R, C}, true);
   return gemm_rm(c, false, true, R, C, C, dZ, BF, C, proj_w, BF, C, 0.0f, dAttn, BF, C);
 }
@@ -658,14 +700,14 @@ Joins joins(int phase, const metalllmSublayerBuffers* b, const AttentionParams* 
   const mla::Span attn_out = span(b->attn_out, e), proj_w = span(b->proj_w, w);
   Joins j{};
   if (phase == 0) {
-    j.residual = b->hidden && tile_rows_ok(R, C, 1) && rows_apart(b->attn_out, b->proj_w, b->out, R, C) &&
+    j.residual = b->hidden && tile_rows_ok(R, C, kProjForward) && rows_apart(b->attn_out, b->proj_w, b->out, R, C) &&
                  !any_overlap({span(b->residual, e)}, {attn_out, proj_w});
     return j;
   }
   const mla::Span X = span(b->X, e), dOut = span(b->dOut, e), Dsum = span(b->Dsum, (size_t)R * p->NH), dX = span(b->dX, e);
   const mla::Span dQ = span(b->dQ, e), dK = span(b->dK, e), dV = span(b->dV, e);
   const mla::Span dWq = span(b->dQw, w), dWk = span(b->dKw, w), dWv = span(b->dVw, w), dWp = span(b->dProjw, w);
-  j.d = p->D == 64 && tile_rows_ok(R, C, 1) && rows_apart(b->dOut, b->proj_w, b->dAttn, R, C) &&
+  j.d = p->D == 64 && tile_rows_ok(R, C, kProjBackward) && rows_apart(b->dOut, b->proj_w, b->dAttn, R, C) &&
         !any_overlap({Dsum}, {dOut, proj_w});
   j.tiles = grad_dx_apart(b->dX, b->q_w, b->k_w, b->v_w, b->dQ, b->dK, b->dV, R, C) &&
             grad_dw_apart(b->X, b->dQ, b->dK, b->dV, b->dQw, b->dKw, b->dVw, R, C) &&

@@ -79,7 +79,8 @@ def test_weight_gradients(gpu, R, H):
 
 
 @pytest.mark.parametrize("B,T,H,D", [(1, 64, 1, 64), (1, 64, 3, 64), (3, 320, 5, 64), (2, 192, 3, 128), (16, 256, 7, 64),
-                                     (64, 128, 1, 64)])
+                                     (64, 128, 1, 64),
+                                     (40, 256, 6, 64)])  # projForward on tiles, the other row products not
 def test_encoder(gpu, B, T, H, D):
     """Both phases through the encoder against the entry points one by one (bit for bit apart from the
     weight gradients' summation order), and a graph of each against the encoder."""
