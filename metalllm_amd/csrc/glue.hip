@@ -355,9 +355,11 @@ __global__ void __launch_bounds__(1024) ln_bwd_kernel(uint16_t* __restrict__ dZ,
 
 // Workgroups of ln_bwd_kernel: the rows' traffic (6 bytes an element, about 20 GB/s a workgroup)
 // takes t = 6 rows cols / (20e9 n) seconds on n of them and the atomics 34e-9 n; the sum is least at
-// n = 0.094 sqrt(rows cols), and there is one workgroup per CU.
+// n = 0.094 sqrt(rows cols), and there is one workgroup per CU. A step of short rows takes the time of
+// its dependent loads and sums, 1.2 us, which 256 columns' traffic takes too: 12500 x 8 42.0 -> 10.3
+// us, 131072 x 8 122 -> 48.5, 4000 x 32 13.9 -> 7.1, 40000 x 64 28.3 -> 20.9, 4000 x 128 9.0 -> 7.8.
 uint32_t ln_bwd_grid(uint32_t rows, uint32_t cols, int rows_per_step) {
-  const uint32_t n = (uint32_t)(0.094 * std::sqrt((double)rows * cols));
+  const uint32_t n = (uint32_t)(0.094 * std::sqrt((double)rows * std::max(cols, 256u)));
   const uint32_t steps = (rows + rows_per_step - 1) / rows_per_step;
   return std::max<uint32_t>(1, std::min<uint32_t>(steps, std::min<uint32_t>(256, std::max<uint32_t>(n, 16))));
 }

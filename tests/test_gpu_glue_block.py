@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("rows,cols", [(4099, 1032), (1000, 1536), (515, 2056), (33, 3080), (1, 1024), (17, 512),
                                        # workgroups whose ranges of steps differ by one (ln_bwd_deal)
-                                       (3077, 4096), (12281, 64), (12288, 768)])
+                                       (3077, 4096), (12281, 64), (12288, 768),
+                                       # short rows, of which one lane or two hold all
+                                       (12500, 8), (1003, 16), (70001, 24)])
 def test_layernorm_row_split(gpu, rows, cols):
     import metalllm_amd.glue as G
     glue_checks.test_layernorm_forward_backward(gpu, G, rows, cols, 1.0)
