@@ -88,8 +88,8 @@ int computeD(const uint16_t* dO, const uint16_t* O, float* D, const AttentionPar
  * dZ is dO; d and l are computeD's and the forward's outputs. dQ += gradient (fp32, accumulated
  * into as in the reference: zero it first for the plain gradient); dK, dV = gradients (bf16).
  * One launch: dK/dV by key-block owners and dQ by query-block owners, each recomputing the
- * softmax tile it needs. For D = 64 and M = 256 (the reference's own shape), where B*NH fills whole
- * rounds of one pair per CU, a workgroup per (b, head) does both and keeps the dS tiles in LDS (dK,
+ * softmax tile it needs. For D = 64 and M = 128 to 256 (the reference's own shape), where B*NH fills
+ * rounds of one pair per CU (nearly full ones, four at M = 128 and two at 192), a workgroup per (b, head) does both and keeps the dS tiles in LDS (dK,
  * dV bit-identical to the other form's, dQ equal up to fp32 summation order). */
 int flashAttentionBackward(const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
                            const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,

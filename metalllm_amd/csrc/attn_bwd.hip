@@ -15,11 +15,11 @@ __global__ void __launch_bounds__(256, (D == 64 && !DS) ? 3 : 2) bwd_kernel(BwdA
   bwd_body<D, DS>(smem, (int)blockIdx.x, a);
 }
 
-// Short sequences (D = 64, T = 256, the reference's own length, where the pairs fill whole rounds:
-// backward_is_short): one persistent workgroup of 8 waves per CU takes (b,h) pairs in turn and does
-// each pair's whole backward, in one launch and without a workspace. LDS holds all query tiles of
-// the pair (bwd_kernel's stage layout, one stage per tile), the pair's K rows and the dS tiles of
-// one query tile.
+// Short sequences (D = 64, T <= 256, the reference's own length, where the pairs nearly fill their
+// rounds: backward_is_short; and outputs in inputs' memory): one persistent workgroup of 8 waves per
+// CU takes (b,h) pairs in turn and does each pair's whole backward, in one launch and without a
+// workspace. LDS holds all query tiles of the pair (bwd_kernel's stage layout, one stage per tile),
+// the pair's K rows and the dS tiles of one query tile.
 //   * Step qt (all waves in step): wave w owns one 32-key group and, when the group lies at or
 //     below query tile qt, runs the DkdvWave step on it and leaves its dS tile in LDS (the
 //     workspace's layout, swizzled as the dQ-from-dS kernel's copies are). Waves w and w + 4

@@ -61,12 +61,20 @@ hipError_t launch_backward_dq(const BwdArgs& a, int D, bool accumulate, hipStrea
 hipError_t launch_backward_dqs(const BwdArgs& a, int D, hipStream_t s); // dQ from the stored dS
 // launch_backward (without the dS store) and launch_backward_dq in one launch, the same results
 hipError_t launch_backward_both(const BwdArgs& a, int D, bool accumulate, hipStream_t s);
-// Sequences of four query tiles (D = 64, T = 256): dK, dV and dQ of a (b,h) pair by one workgroup
-// per CU, one launch, no workspace; dQ added into (accumulate) or written. It takes 21.5 us for
-// each round of kCus pairs, bwd_both_kernel 0.085-0.089 us a pair (and 10 us at least), so it is the
-// faster one only where its last round is nearly full: 768 pairs 63.6 against 64.7 us, 1536 pairs
-// 129.9 against 136.8, but 6 pairs 19.0 against 10.8, 320 pairs 42.5 against 30.5. At T <= 192 it is
-// nowhere faster by more than 1% (two tiles, 6 to 1536 pairs: 10.6-58.3 against 9.8-57.1 us).
+// Short sequences (D = 64, T <= 256): dK, dV and dQ of a (b,h) pair by one workgroup per CU, one
+// launch, no workspace; dQ added into (accumulate) or written. It takes the same time for each round of
+// kCus pairs, full or not (T = 128, 192, 256: 10.3, 15.7, 21.5 us), and a little for the first;
+// bwd_both_kernel takes a time per pair, which grows by a fifth where a call's tensors exceed what the
+// caches hold (from 350000 rows on), as it reads the inputs twice. So this kernel is the faster one
+// where its rounds are nearly full, by more the larger the call. us, this kernel against the other,
+// dQ written / added into:
+//   T = 256: 240 pairs 24.9 / 25.6 against 26.3 / 26.5, 320 42.0 / 43.1 against 31.9 / 33.5, 768 65.2 /
+//     66.6 against 66.2 / 72.0, 1536 142 / 150 against 158 / 169, 3072 273 / 287 against 325 / 354
+//   T = 192: 448 33.0 / 33.9 against 32.9 / 34.5, 512 34.4 / 35.1 against 36.6 / 39.1, 640 46.6 / 48.0 against
+//     44.9 / 47.5, 1280 76 / 78 against 84 / 90, 3072 201 / 215 against 246 / 267
+//   T = 128: 768 33.2 / 33.9 against 31.9 / 34.7, 1024 41.7 / 42.7 against 43.4 / 45.1, 2048 79.7 / 82.9 against
+//     79.2 / 85.4, 4096 173 / 184 against 199 / 220
+//   T = 64: 1024 23.9 / 25.0 against 23.3 / 24.5, 6144 176 / 187 against 146 / 169
 // Defined below, at kCus.
 __host__ __device__ inline bool backward_is_short(int T, int D, int pairs);
 // Whether the workspace entry point runs the recomputing kernels (dK/dV without the dS store and dQ
@@ -133,7 +141,10 @@ constexpr int kCus = 256;
 
 __host__ __device__ inline bool backward_is_short(int T, int D, int pairs) {
   const int rounds = (pairs + kCus - 1) / kCus;
-  return D == 64 && T == 256 && pairs * 20 >= 19 * kCus * rounds;
+  const bool large = (int64_t)pairs * T >= 350000;
+  const int fill = T == 256 ? (large ? 88 : 93) : T == 192 ? (large ? 85 : 90) : (large ? 90 : 95);  // percent
+  return D == 64 && T >= 128 && T <= 256 && rounds >= (T == 256 ? 1 : T == 192 ? 2 : 4) &&
+         (int64_t)pairs * 100 >= (int64_t)fill * kCus * rounds;
 }
 
 // Item k of workgroup `bid` of a persistent grid of `grid` workgroups over npairs x nblk

@@ -1,12 +1,12 @@
 """The backward's launches by shape: dK/dV and dQ in one launch (whole grids resident, with the dQ
 blocks of every second row of ids reversed, by XCD octets and not; more workgroups than are
-resident), the stored-dS path at D = 128 beyond two blocks per CU, and the fused kernel of whole
-rounds of T = 256 pairs. Every shape goes through both entry points against the oracle at the bars of
+resident), the stored-dS path at D = 128 beyond two blocks per CU, and the fused kernel of nearly
+full rounds of pairs at T = 128 to 256. Every shape goes through both entry points against the oracle at the bars of
 test_gpu_parity.py (outputs start as NaN where they are written in full)."""
 import numpy as np
 import pytest
 
-from tests.attn_case import gpu_backward, gpu_compute_d, gpu_forward, make_inputs
+from tests.attn_case import gpu_backward, gpu_compute_d, gpu_forward, make_inputs, to_gpu
 from tests.test_gpu_parity import check_case
 
 pytestmark = pytest.mark.gpu
@@ -21,11 +21,38 @@ pytestmark = pytest.mark.gpu
     (23, 256, 8, 128, 1),    # 368 blocks: below the line of T < 512 (384)
     (25, 256, 8, 128, 1),    # 400 blocks: above it
     (9, 576, 13, 128, 1),    # 585 blocks: dS stored, four-tile ring, last item 1 of 4 tiles
-    (122, 256, 2, 64, 1),    # 244 pairs: the fused T = 256 kernel, one round 95% full
-    (121, 256, 2, 64, 1),    # 242 pairs: below that line
+    (122, 256, 2, 64, 1),    # 244 pairs: the fused kernel, one round 95% full
+    (121, 256, 2, 64, 1),    # 242 pairs: the same, 94.5%
+    (119, 256, 2, 64, 1),    # 238 pairs: below the line
+    (128, 192, 4, 64, 1),    # 512 pairs: the fused kernel, three query tiles, two full rounds
+    (205, 128, 5, 64, 1),    # 1025 pairs: 82% of five rounds, below the line
+    (244, 128, 5, 64, 1),    # 1220 pairs: the fused kernel, two query tiles, the last of five rounds partly full
 ])
 def test_launch_forms(gpu, B, T, H, D, b_end):
     check_case(gpu, B, T, H, D, 1.0, 211, b_end=b_end)
+
+
+@pytest.mark.parametrize("B,T,H", [(247, 256, 2), (241, 192, 2), (244, 128, 5)])
+def test_fused_kernel_adds(gpu, B, T, H):
+    """flashAttentionBackward's contract in the fused kernel, more pairs than one round: dQ starts at
+    values that are not zero and ends at those plus the gradient (one fp32 addition each)."""
+    import torch
+    import metalllm_amd as M
+    import metalllm_amd.attention as A
+    assert A.backward_route(B, T, H, 64, False) == A.FUSED
+    q, k, v, g = (to_gpu(x, gpu) for x in make_inputs(B, T, H, 64, 213))
+    out, lse = M.attention_forward(q, k, v)
+    Dv = torch.empty_like(lse)
+    M.computeD(g, out, Dv)
+    ws = torch.empty((M.workspace_bytes(B, T, H, 64),), dtype=torch.uint8, device=gpu)
+    dQ, dK, dV = torch.full((B, T, H, 64), float("nan"), device=gpu), torch.empty_like(q), torch.empty_like(q)
+    M.flashAttentionBackwardWorkspace(g, Dv, lse, q, k, v, dQ, dK, dV, ws)
+    old = torch.randn((B, T, H, 64), generator=torch.Generator(gpu).manual_seed(5), device=gpu)
+    dQ2, dK2, dV2 = old.clone(), torch.empty_like(q), torch.empty_like(q)
+    M.flashAttentionBackward(g, Dv, lse, q, k, v, dQ2, dK2, dV2)
+    torch.cuda.synchronize()
+    assert torch.equal(dQ2, old + dQ)
+    assert torch.equal(dK, dK2) and torch.equal(dV, dV2)
 
 
 def test_short_kernel_agrees_with_both(gpu):
