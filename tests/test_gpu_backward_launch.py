@@ -32,6 +32,43 @@ def test_launch_forms(gpu, B, T, H, D, b_end):
     check_case(gpu, B, T, H, D, 1.0, 211, b_end=b_end)
 
 
+# D = 128 beyond the lines of the joint launch: dK/dV storing dS, then the dQ ring of two query tiles an
+# item (T < 512) or four, with last items of one to all of them
+STORED = [(193, 64, 2), (97, 192, 2), (65, 320, 2), (65, 448, 2), (49, 256, 8), (17, 512, 8), (15, 576, 7), (26, 640, 4),
+          (22, 704, 4)]
+
+
+@pytest.mark.parametrize("B,T,H", STORED)
+def test_stored_ds(gpu, B, T, H):
+    import metalllm_amd.attention as A
+    assert A.backward_route(B, T, H, 128, True) == A.STORED
+    check_case(gpu, B, T, H, 128, 1.5 if T == 320 else 1.0, 214, b_end=1)
+
+
+@pytest.mark.parametrize("B,T,H", [(65, 448, 2), (17, 512, 8)])
+def test_stored_parts_equal_the_entry_point(gpu, B, T, H):
+    """The bench hook's parts 2 and 3 where they store dS: flashAttentionBackwardWorkspace bit for bit."""
+    import torch
+    import metalllm_amd as M
+    q, k, v, g = (to_gpu(x, gpu) for x in make_inputs(B, T, H, 128, 215))
+    out, lse = M.attention_forward(q, k, v)
+    Dv = torch.empty_like(lse)
+    M.computeD(g, out, Dv)
+    res = []
+    for parts in (False, True):
+        ws = torch.full((M.workspace_bytes(B, T, H, 128),), 0x7F, dtype=torch.uint8, device=gpu)
+        r = [torch.full(q.shape, float("nan"), device=gpu), torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))]
+        if parts:
+            M.backward_part(2, g, Dv, lse, q, k, v, *r, workspace=ws)
+            assert torch.isnan(r[0]).all()  # dQ comes from the stored dS alone
+            M.backward_part(3, g, Dv, lse, q, k, v, *r, workspace=ws)
+        else:
+            M.flashAttentionBackwardWorkspace(g, Dv, lse, q, k, v, *r, ws)
+        res.append(r)
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("B,T,H", [(247, 256, 2), (241, 192, 2), (244, 128, 5)])
 def test_fused_kernel_adds(gpu, B, T, H):
     """flashAttentionBackward's contract in the fused kernel, more pairs than one round: dQ starts at

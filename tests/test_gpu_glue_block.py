@@ -23,7 +23,10 @@ def test_layernorm_row_split(gpu, rows, cols):
 
 
 @pytest.mark.parametrize("B,T,H,C", [(1, 64, 1, 64), (3, 192, 6, 384), (2, 64, 12, 768), (1, 128, 20, 1280), (1, 64, 20, 2560),
-                                     (8, 1024, 12, 768), (3, 320, 5, 320), (2, 192, 3, 384)])
+                                     (8, 1024, 12, 768), (3, 320, 5, 320), (2, 192, 3, 384),
+                                     # ln1's backward in ranges of 3 and 4 steps that end apart (ln_bwd_deal), its rows
+                                     # by one wave and by two; the last with ranges that differ by one
+                                     (48, 256, 12, 768), (32, 256, 24, 1536), (49, 256, 12, 768)])
 def test_block_ends(gpu, B, T, H, C):
     """Also computeD and the residual add where the projections' tiles do them (D = 64; residual at
     every D), against the public calls on the encoder's own dAttn, attn_out and out."""

@@ -7,7 +7,7 @@ max-abs relative to max |grad|; computeD bit-exact (the reference's lane-strided
 oracle's butterfly model of simd_sum); causal-mask and index logic exact (row 0 of O equals row 0
 of V bit for bit; with V one-hot every future weight is exactly zero). Both backward entry points
 are checked: flashAttentionBackward (which adds into dQ, as the reference's atomics do) and
-flashAttentionBackwardWorkspace (the stored-dS path, which writes dQ); their dK/dV must also be
+flashAttentionBackwardWorkspace (which writes dQ; from stored dS where test_gpu_backward_launch.py says); their dK/dV must also be
 identical to each other, their dQ equal within 1e-5 of max |dQ| (fp32 summation order).
 """
 import ctypes
@@ -71,10 +71,12 @@ CASES = [
     (1, 192, 3, 128, 1.5, 14),    # T not a multiple of 128/256, odd head count
     (1, 64, 1, 64, 1.0, 15),      # a single tile
     (3, 320, 1, 64, 1.0, 16),     # 5 tiles, B*H not a multiple of 8
-    (4, 448, 2, 128, 1.0, 17),    # 8 pairs: XCD-affine two-tile dQ ring (T < 512), 7 tiles
-    (2, 576, 4, 128, 1.0, 18),    # 8 pairs: XCD-affine four-tile dQ ring, last item 1 of 4 tiles
-    (2, 128, 3, 64, 1.5, 19),     # short-sequence backward (one workgroup per pair), two tiles, peaky
-    (1, 192, 5, 64, 1.0, 20),     # short-sequence backward, three tiles (idle waves in both phases)
+    # few pairs: both backward entry points run the joint launch (the stored-dS rings and the fused
+    # kernel, which take many, are in test_gpu_backward_launch.py)
+    (4, 448, 2, 128, 1.0, 17),    # 8 pairs: XCD-affine, 7 tiles
+    (2, 576, 4, 128, 1.0, 18),    # 8 pairs: XCD-affine, 9 tiles
+    (2, 128, 3, 64, 1.5, 19),     # two tiles, peaky
+    (1, 192, 5, 64, 1.0, 20),     # three tiles
 ]
 
 
@@ -84,8 +86,8 @@ def test_forward_backward_parity(gpu, B, T, H, D, s, seed):
 
 
 def _sweep_cases(n=14, seed=2024):
-    """Seeded shape sweep: T every multiple of 64 up to 640 (short fused backward and persistent
-    forward at T <= 256, both dQ rings above), odd and even head and batch counts (pair counts
+    """Seeded shape sweep: T every multiple of 64 up to 640 (few pairs: the persistent forward and the
+    joint backward), odd and even head and batch counts (pair counts
     that are and are not multiples of 8), both head sizes and both Q/K scales."""
     rng = np.random.default_rng(seed)
     cases = []
@@ -268,10 +270,9 @@ def test_backward_dq_contract(gpu):
     into a caller-zeroed buffer, attention.metal:292-296, model.h:549): with dQ prefilled, the
     result is prefill + gradient, each element one fp32 add of the zero-start result. It writes dK
     and dV in full (stale contents ignored). flashAttentionBackwardWorkspace writes all three in
-    full, whatever the stale contents of its outputs or of the workspace. D = 64 at T <= 256 runs
-    the fused short-sequence kernel; T = 512 at D = 64 and both D = 128 shapes run the recomputing
-    dQ kernel's read-add-write. At D = 64 the workspace entry point stores no dS (the fused kernel,
-    or the recomputing kernels with dQ written), so its dQ equals the zero-start gradient bit for
+    full, whatever the stale contents of its outputs or of the workspace. All
+    shapes here run the joint launch (the fused kernel's additions are in test_gpu_backward_launch.py).
+    At D = 64 the workspace entry point stores no dS, so its dQ equals the zero-start gradient bit for
     bit."""
     import torch
     import metalllm_amd as M
@@ -421,7 +422,8 @@ def test_config3_against_plain_fp32_order(gpu):
 
 def test_backward_parts_equal_flash_attention_backward(gpu):
     """The bench hook: part 0 (dK/dV kernel) then part 1 (dQ kernel) is flashAttentionBackward, and
-    part 2 then part 3 is flashAttentionBackwardWorkspace, bit for bit."""
+    part 2 then part 3 is flashAttentionBackwardWorkspace, bit for bit (here both the joint launch; parts
+    2 and 3 with the dS store are in test_gpu_backward_launch.py)."""
     import torch
     import metalllm_amd as M
     q, k, v, g = make_inputs(2, 512, 3, 128, 41)

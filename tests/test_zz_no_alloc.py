@@ -38,7 +38,13 @@ def _run(gpu, B, T, H, D, seed):
 
 
 def test_no_alloc_backward_matches_workspace_backward(gpu):
-    # D = 128 stores dS tiles in the array: 53.5 MB of them (near its 64 MiB), then a smaller input
+    # D = 128 beyond two blocks of 128 rows per CU stores dS tiles in the array: 660 blocks, 48.7 MB (of
+    # its 64 MiB), then a smaller input
+    import metalllm_amd.attention as A
+    for B, seed in ((33, 65), (26, 66)):
+        assert A.backward_route(B, 512, 5, 128, True) == A.STORED
+        _run(gpu, B, 512, 5, 128, seed)
+    # fewer blocks: recomputed, though the nominal size counts (53.5 MB, then a smaller input)
     _run(gpu, 4, 1024, 12, 128, 61)
     _run(gpu, 2, 512, 4, 128, 62)
     # D = 64 stores no tiles (T <= 256: the fused short backward; longer: the recomputing kernels):
