@@ -7,10 +7,11 @@
 namespace mla {
 
 // D = 64 without the dS store: three workgroups per CU (168 VGPRs, a few spilled outside the
-// product loop), 6-8% faster than two. D = 64 with the dS store: two workgroups per CU and the
-// fp32 dK/dV state. D = 128 needs its 244-253 VGPRs and runs two.
+// product loop), 6-8% faster than two. D = 128 needs its 244-253 VGPRs and runs two. Without the dS
+// store these run where outputs are in inputs' memory (the joint launch needs them apart), and as parts.
 template <int D, bool DS>
-__global__ void __launch_bounds__(256, (D == 64 && !DS) ? 3 : 2) bwd_kernel(BwdArgs a) {
+__global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_kernel(BwdArgs a) {
+  static_assert(D == 128 || !DS, "no dS is stored at D = 64");
   __shared__ __attribute__((aligned(1024))) unsigned char smem[BwdCfg<D>::SMEM];
   bwd_body<D, DS>(smem, (int)blockIdx.x, a);
 }
@@ -207,7 +208,6 @@ hipError_t launch_backward(const BwdArgs& a, int D, hipStream_t s) {
   const int nkb = (a.T + kBwdBlockN - 1) / kBwdBlockN;
   const dim3 grid((unsigned)(a.B * a.H * nkb));
   if (a.dS) {
-    // at D = 64 the workspace entry point stores no dS (workspace_recomputes, backward_is_short)
     if (D == 64) return hipErrorInvalidValue;
     hipLaunchKernelGGL((bwd_kernel<128, true>), grid, dim3(256), 0, s, a);
   } else {

@@ -1,5 +1,5 @@
-// attn_bwd_dq.hip -- the kernel of flashAttentionBackward's dQ half (attn_bwd_dq.hpp holds a
-// workgroup's body).
+// attn_bwd_dq.hip -- the kernel of flashAttentionBackward's dQ half by itself (attn_bwd_dq.hpp holds a
+// workgroup's body): the second of two launches where outputs are in inputs' memory, and a part.
 #include "attn_bwd_dq.hpp"
 
 namespace mla {

@@ -13,8 +13,8 @@
 // 1 KB chunk rows s = 0..3, each 64 lanes x 16 bytes: lane l = key32 + 32h carries the 8 values
 // of key 32hw + key32 at query positions p = 32h + 8s + e (e = 0..7), and position p is query
 // q(p) = 32t + 8j + 4h + i of the tile with p % 32 = 16t + 4j + i. That is the order the dK/dV
-// kernel holds dS in its accumulators, so it stores with four full 16-byte writes per lane. At
-// D = 64 the tiles hold 8 dS (the power-of-two scale 1/8 is applied to dQ when it is stored).
+// kernel holds dS in its accumulators, so it stores with four full 16-byte writes per lane. (D = 128
+// only: at D = 64 recomputing dS is faster, and no kernel stores it.)
 //
 // Work split: an item is QT query tiles (64 rows each) of one (b, h); wave w of the workgroup
 // computes dQ^T of query tile qt0 + w/2 for the d half w%2, over key tiles 0 .. qt0 + QT - 1.
@@ -31,7 +31,7 @@
 // LDS layout, no padding: K rows and dS chunk rows are XOR-swizzled in 16-byte chunks so that
 // the transposing reads are conflict-free (the 4 rows x 64 bytes that 32 lanes of one
 // ds_read_b64_tr_b16 touch fall in distinct banks). K row r, LDS chunk p holds K chunk
-// p ^ kx(r), kx(r) = 4(r % 4) (D = 128, 16 chunks a row) or 4((r / 2) % 2) (D = 64, 8 chunks);
+// p ^ kx(r), kx(r) = 4(r % 4) (16 chunks a row);
 // dS chunk row c, LDS slot s holds the row's slot s ^ 4(c % 4). A copy lane fetches the global
 // chunk that belongs at its LDS slot, so the copies stay whole 16-byte transfers within a row.
 //
@@ -46,7 +46,7 @@
 // the same operand registers as dQ^T = K^T.dS^T, the same sums bit for bit) so that a lane holds
 // one d of 16 rows: each 4-byte store writes 32 consecutive d of a row per half wave, whole
 // 128-byte lines (with dQ^T each 16-byte store wrote 32-byte pieces of 32 rows; c3 1.047 ->
-// 1.015 ms, c2 0.113 -> 0.109 ms). The vmcnt waits saturate at 63: with 64 stores per item a
+// 1.015 ms). The vmcnt waits saturate at 63: with 64 stores per item a
 // wait may also cover a few of them, which only waits longer.
 #include <algorithm>
 #include <atomic>
@@ -108,9 +108,7 @@ template <int D, int QT, int NSTAGE>
 __global__ void __launch_bounds__(128 * QT, (NSTAGE * (128 * D + 8192 * QT) <= 80 * 1024 ? 2 : 1))
 dqs_kernel(BwdArgs a) {  // (THREADS, WG_PER_CU of DqsCfg)
   using C = DqsCfg<D, QT, NSTAGE>;
-  // the stored dS tiles of D = 64 hold 8 dS (the dK/dV kernel folds the power-of-two scale 1/8
-  // into the stores of dK and dQ): dQ = (sum of 8 dS . K) / 8, exact
-  constexpr float kDsUnit = D == 64 ? 0.125f : 1.0f;
+  static_assert(D == 128, "K rows of 16 chunks; dS unscaled");
   static_assert(C::THREADS == 128 * QT && C::WG_PER_CU == (NSTAGE * C::STAGE <= 80 * 1024 ? 2 : 1), "launch bounds");
   __shared__ __attribute__((aligned(1024))) unsigned char smem[C::NSTAGE * C::STAGE];
 
@@ -141,7 +139,7 @@ dqs_kernel(BwdArgs a) {  // (THREADS, WG_PER_CU of DqsCfg)
     const int b = pair / a.H, hd = pair - b * a.H;
     return ((size_t)b * a.T * a.H + hd) * D;
   };
-  auto kx = [](int r) { return D == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
+  auto kx = [](int r) { return 4 * (r & 3); };
 
   // copies of a stage: K instructions wave + WAVES*j (LDS slot L = 64*ins + lane: row L / KCH,
   // chunk L % KCH); dS instructions d = wave + WAVES*j, tile d / 8, chunk row d % 8
@@ -298,7 +296,7 @@ dqs_kernel(BwdArgs a) {  // (THREADS, WG_PER_CU of DqsCfg)
           const int x = 8 * (r >> 2) + 4 * h + (r & 3);
           const int qin = 32 * (x >> 4) + 8 * ((x >> 2) & 3) + 4 * nb + (x & 3);
 #pragma unroll
-          for (int mm = 0; mm < C::MB; ++mm) dQg[(size_t)qin * rs + 32 * mm] = acc[mm][nb][r] * kDsUnit;
+          for (int mm = 0; mm < C::MB; ++mm) dQg[(size_t)qin * rs + 32 * mm] = acc[mm][nb][r];
         }
       s1 = true;
     }
@@ -324,6 +322,7 @@ static hipError_t launch_ring(const BwdArgs& a, int cus, hipStream_t s) {
 }
 
 hipError_t launch_backward_dqs(const BwdArgs& a, int D, hipStream_t s) {
+  if (D != 128) return hipErrorInvalidValue;
   // CU count of the current device (cached per device; the query does not touch the stream)
   static std::atomic<int> cu_cache[64];
   int dev = 0;
@@ -336,8 +335,6 @@ hipError_t launch_backward_dqs(const BwdArgs& a, int D, hipStream_t s) {
   }
   // four query tiles per item from 512 keys on (T = 256 has a single such item per pair)
   const bool deep = a.T >= 512;
-  if (D == 64)
-    return deep ? launch_ring<64, 4, 3>(a, cus, s) : launch_ring<64, 2, 2>(a, cus, s);
   return deep ? launch_ring<128, 4, 3>(a, cus, s) : launch_ring<128, 2, 2>(a, cus, s);
 }
 
