@@ -5,18 +5,20 @@ flashAttentionBackward) on one MI355X, through the C ABI.
 
 One step = flashAttentionForward + computeD + the backward over one batch of synthetic bf16 inputs
 already resident in HBM (the reference's per-layer sequence, model.h:459-473, 639-665). The
-backward is flashAttentionBackwardWorkspace (dK/dV kernel storing dS into a device workspace, then
-dQ = dS.K; workspace allocated once, outside the timed region, like the other buffers); the
-recomputing flashAttentionBackward is timed beside it ("bwd_recompute"). Prints ONE JSON line.
+backward is flashAttentionBackwardWorkspace (at D = 128 and many blocks a dK/dV kernel storing dS
+into a device workspace, then dQ = dS.K; workspace allocated once, outside the timed region, like the
+other buffers); the recomputing flashAttentionBackward is timed beside it ("bwd_recompute"). Prints
+ONE JSON line.
 FLOPs use the causal FlashAttention convention (half of dense): fwd 2*B*H*T^2*D, bwd
 5*B*H*T^2*D, step 7*B*H*T^2*D.
 
-The roofline object describes the dominant kernel, the dK/dV kernel (mla::bwd_kernel with the dS
-store; the bench launches the backward's two kernels through metalllmAttnBackwardPart so that
-each has its own events): its algorithmic FLOPs per launch (4 causal products: S, dP, dV, dK) over
-its average launch time measured with HIP events on the launch stream, against MI355X dense bf16
-matrix peak. roofline_dq does the same for the HBM-bound dQ kernel (bytes of dS, K and dQ per
-launch against 8 TB/s). cpu_baseline times the CPU oracle (the scalar C++ transcription of the
+The roofline object describes the backward's dominant kernel. Where the entry point runs two (D =
+128, many blocks) that is the dK/dV kernel (mla::bwd_kernel with the dS store; steps of their own
+launch the two through metalllmAttnBackwardPart so that each has its events): its algorithmic FLOPs
+per launch (4 causal products: S, dP, dV, dK) over its average launch time measured with HIP events on
+the launch stream, against MI355X dense bf16 matrix peak; roofline_dq does the same for the HBM-bound
+dQ kernel (bytes of dS, K and dQ per launch against 8 TB/s). Elsewhere it is the one kernel that
+computes dK, dV and dQ. cpu_baseline times the CPU oracle (the scalar C++ transcription of the
 reference math, oracle/attn_oracle.cpp) on a bounded sample of the same workload on this host's
 cores.
 """
@@ -228,11 +230,12 @@ def step_bound_ms(B, H, T, D):
 
 def run_core(cfg_id, steps, warmup, calibrate_copy=False):
     """Times the attention core of one config (fwd + computeD + backward, inputs resident in HBM).
-    Two step kinds: the headline step with flashAttentionBackwardWorkspace (parts 2 and 3) and the
-    reference-contract step with flashAttentionBackward (parts 0 and 1, into a zeroed dQ, the
-    memset included). Returns the per-kernel event spans and both steps' spans."""
+    Two step kinds: the headline step with flashAttentionBackwardWorkspace and the
+    reference-contract step with flashAttentionBackward (into a zeroed dQ, the memset included).
+    Returns the per-kernel event spans and both steps' spans."""
     import torch
     import metalllm_amd as M
+    from metalllm_amd.attention import FUSED, JOINT, STORED, TWO, backward_route
 
     B, H, T, D, qk_scale, desc = CONFIGS[cfg_id]
     dev = torch.device("cuda:0")
@@ -258,52 +261,61 @@ def run_core(cfg_id, steps, warmup, calibrate_copy=False):
     stream = torch.cuda.current_stream()
     p = M.AttentionParams.of(B, T, H, D)
 
-    # flashAttentionBackwardWorkspace == part 2 (dK/dV kernel + dS store) then part 3 (dQ from dS);
-    # flashAttentionBackward == part 0 then part 1. The bench launches the parts itself so that
-    # each kernel is timed by its own events. The workspace path writes dQ in full; the
-    # recomputing path adds into dQ (the reference's contract), so its steps zero dQ first.
+    # Both kinds of step call the entry points. Where one runs two kernels, the steps that time the
+    # phases launch them as the parts it consists of, with a marker between. The workspace path writes
+    # dQ in full; the recomputing path adds into dQ (the reference's contract), so its steps zero dQ.
     # ev: None (untimed), 5 events (a marker before, between and after the kernels: the phase
     # spans) or 2 events (start and end only: the step span, free of the markers' own cost,
     # which is a few microseconds each)
-    def step(ev=None, parts=(2, 3)):
-        flush.fill_(parts[0])
-        mark = (lambda i: ev[i].record(stream)) if ev is not None and len(ev) == 5 else (lambda i: None)
+    addresses = [t.data_ptr() for t in (dO, Dv, lse, q, k, v, dQ, dK, dV)]
+    route = {w: backward_route(B, T, H, D, w, addresses) for w in (True, False)}
+
+    def step(ev=None, workspace=True):
+        flush.fill_(int(workspace))
+        marked = ev is not None and len(ev) == 5
+        mark = (lambda i: ev[i].record(stream)) if marked else (lambda i: None)
         if ev is not None:
             ev[0].record(stream)
         M.flashAttentionForward(q, k, v, out, lse, stream, p)
         mark(1)
         M.computeD(dO, out, Dv, stream, p)
         mark(2)
-        if parts[0] == 0:
+        if not workspace:
             dQ.zero_()  # the memset the reference's caller does (model.h:549), timed with the backward
-        M.backward_part(parts[0], dO, Dv, lse, q, k, v, dQ, dK, dV, stream, p, workspace=ws)
-        mark(3)
-        M.backward_part(parts[1], dO, Dv, lse, q, k, v, dQ, dK, dV, stream, p, workspace=ws)
+        if marked and route[workspace] in (TWO, STORED):
+            first = 2 if workspace else 0
+            M.backward_part(first, dO, Dv, lse, q, k, v, dQ, dK, dV, stream, p, workspace=ws)
+            mark(3)
+            M.backward_part(first + 1, dO, Dv, lse, q, k, v, dQ, dK, dV, stream, p, workspace=ws)
+        elif workspace:
+            M.flashAttentionBackwardWorkspace(dO, Dv, lse, q, k, v, dQ, dK, dV, ws, stream, p)
+        else:
+            M.flashAttentionBackward(dO, Dv, lse, q, k, v, dQ, dK, dV, stream, p)
         if ev is not None:
             ev[-1].record(stream)
 
-    def timed_steps(parts, n, nev):
+    def timed_steps(workspace, n, nev):
         evs = [[torch.cuda.Event(enable_timing=True) for _ in range(nev)] for _ in range(n)]
         for e in evs:
-            step(e, parts=parts)
+            step(e, workspace)
         torch.cuda.synchronize()
         return evs
 
     # the reference-contract step (flashAttentionBackward): its own warmup, phase and step spans
     n_rc = max(3, steps // 4)
     for _ in range(2):
-        step(parts=(0, 1))
-    rc_events = timed_steps((0, 1), n_rc, 5)
-    rc_plain = timed_steps((0, 1), n_rc, 2)
+        step(workspace=False)
+    rc_events = timed_steps(False, n_rc, 5)
+    rc_plain = timed_steps(False, n_rc, 2)
 
     for _ in range(warmup):
         step()
     torch.cuda.synchronize()
     # phase spans: steps with markers between the kernels
-    events = timed_steps((2, 3), steps, 5)
+    events = timed_steps(True, steps, 5)
     # headline: the same steps with one event pair each
     t0 = time.perf_counter()
-    plain = timed_steps((2, 3), steps, 2)
+    plain = timed_steps(True, steps, 2)
     wall = time.perf_counter() - t0
 
     if calibrate_copy:
@@ -314,12 +326,14 @@ def run_core(cfg_id, steps, warmup, calibrate_copy=False):
         torch.cuda.synchronize()
 
     span = lambda a, b, evs=events: sorted(e[a].elapsed_time(e[b]) for e in evs)
+    two = lambda w: route[w] in (TWO, STORED)  # kv and dq: the two kernels, None where one does both
     res = {
         "shape": (B, H, T, D, qk_scale, desc), "ws_bytes": ws_bytes,
-        "fwd": span(0, 1), "cd": span(1, 2), "kv": span(2, 3), "dq": span(3, 4), "bwd": span(2, 4),
+        "kernel": {FUSED: "fused", JOINT: "joint", TWO: "two", STORED: "stored"}[route[True]],
+        "fwd": span(0, 1), "cd": span(1, 2), "kv": span(2, 3) if two(True) else None,
+        "dq": span(3, 4) if two(True) else None, "bwd": span(2, 4),
         "marked": span(0, 4), "step": span(0, 1, plain), "wall_ms": wall * 1e3 / steps,
-        "rc_kv": span(2, 3, rc_events), "rc_dq": span(3, 4, rc_events), "rc_bwd": span(2, 4, rc_events),
-        "rc_step": span(0, 1, rc_plain),
+        "rc_bwd": span(2, 4, rc_events), "rc_step": span(0, 1, rc_plain),
     }
     del q, k, v, dO, flush, out, lse, Dv, dQ, dK, dV, ws
     torch.cuda.empty_cache()
@@ -328,6 +342,10 @@ def run_core(cfg_id, steps, warmup, calibrate_copy=False):
 
 def med(xs):
     return xs[len(xs) // 2]
+
+
+def med4(xs):
+    return None if xs is None else round(med(xs), 4)
 
 
 def core_summary(cfg_id, r):
@@ -349,8 +367,8 @@ def core_summary(cfg_id, r):
                           "over fwd, computeD and bwd"},
         "frac_of_bound": round(bound / ms, 4),
         "phases_ms_median": {"fwd": round(med(r["fwd"]), 4), "computeD": round(med(r["cd"]), 4),
-                             "bwd": round(med(r["bwd"]), 4), "bwd_dkdv": round(med(r["kv"]), 4),
-                             "bwd_dq": round(med(r["dq"]), 4)},
+                             "bwd": round(med(r["bwd"]), 4), "bwd_dkdv": med4(r["kv"]), "bwd_dq": med4(r["dq"])},
+        "bwd_kernels": r["kernel"],
         "ref_contract_step": {"ms_per_step": round(rc_ms, 4),
                               "tflops": round((ff + fb) / (rc_ms * 1e-3) / 1e12, 2),
                               "bwd_ms_median": round(med(r["rc_bwd"]), 4)},
@@ -407,61 +425,48 @@ def main():
     ms_per_step = med(r["step"])
     marked_ms = med(r["marked"])
     value = (ff + fb) / (ms_per_step * 1e-3) / 1e12
-    # dominant kernel: the dK/dV kernel (4 products: S, dP, dV = P^T dO, dK = dS^T Q)
-    kv_avg = avg(kv_ms)
-    achieved = 4.0 * unit / (kv_avg * 1e-3) / 1e12
-    # dQ kernel from the stored dS: reads every dS tile once, K (once per 128-query block, from L2
-    # after the first), writes dQ fp32 once; algorithmic bytes = dS + K + dQ
     bthd = B * T * H * D
-    dq_bytes = ws_bytes + 2 * bthd + 4 * bthd
-    dq_avg = avg(dq_ms)
-    rc_kv, rc_dq, rc_bwd = r["rc_kv"], r["rc_dq"], r["rc_bwd"]
-
-    if D == 64 and T <= 256:
-        # short sequences: one fused kernel (part 2) computes dK, dV and dQ without the workspace
-        # (part 3 launches nothing); at T = 256 the backward is HBM-bound (5T/16 FLOP per byte)
+    bwd_avg = avg(bwd_ms)
+    roofline_dq = None
+    if r["kernel"] == "fused":
+        # short sequences: one fused kernel computes dK, dV and dQ without the workspace; at T = 256 the
+        # backward is HBM-bound (5T/16 FLOP per byte)
         bwd_bytes = 16 * bthd + 8 * B * H * T
         roofline = {
             "kernel": "fused short-sequence backward (mla::bwd_short_kernel<false>: dK, dV and dQ)",
             "bound": "hbm",
-            "achieved": round(bwd_bytes / (kv_avg * 1e-3) / 1e9, 1),
+            "achieved": round(bwd_bytes / (bwd_avg * 1e-3) / 1e9, 1),
             "peak": PEAK_HBM_GBS,
             "unit": "GB/s",
-            "frac": round(bwd_bytes / (kv_avg * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
+            "frac": round(bwd_bytes / (bwd_avg * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
             "traffic": traffic_from_profiles(args.config, "bwd_short"),
             "algorithmic_bytes": bwd_bytes,
-            "tflops": round(5.0 * unit / (kv_avg * 1e-3) / 1e12, 2),
-            "avg_ms": round(kv_avg, 4),
+            "tflops": round(5.0 * unit / (bwd_avg * 1e-3) / 1e12, 2),
+            "avg_ms": round(bwd_avg, 4),
         }
-        roofline_dq = None
-    elif D == 64:
-        # the workspace entry point runs the recomputing kernels at D = 64 (no dS stored): dK/dV
-        # (4 products: S, dP, dV, dK) and dQ written (3 products: S, dP, dQ)
+    elif r["kernel"] == "joint":
+        # dK/dV (4 products: S, dP, dV, dK) and dQ (S, dP, dQ), no dS stored
+        executed = 7.0 * unit / (bwd_avg * 1e-3) / 1e12
         roofline = {
-            "kernel": "backward dK/dV kernel without the dS store (mla::bwd_kernel<64, false>; at D = 64 "
-                      "the workspace entry point recomputes dS instead of storing it)",
+            "kernel": "backward dK/dV and dQ in one launch, both recomputing S, dP and dS (mla::bwd_both_kernel)",
             "bound": "mfma",
-            "achieved": round(achieved, 2),
+            "achieved": round(executed, 2),
             "peak": PEAK_BF16_TFLOPS,
             "unit": "TFLOP/s",
-            "frac": round(achieved / PEAK_BF16_TFLOPS, 4),
+            "frac": round(executed / PEAK_BF16_TFLOPS, 4),
             "traffic": None,
-            "algorithmic_bytes": 12 * bthd + 8 * B * H * T,
-            "avg_ms": round(kv_avg, 4),
-        }
-        dq_exec = 3.0 * unit / (dq_avg * 1e-3) / 1e12
-        roofline_dq = {
-            "kernel": "backward dQ kernel recomputing S, dP and dS, dQ written (mla::bwd_dq_kernel<64, false>)",
-            "bound": "mfma",
-            "achieved": round(dq_exec, 2),
-            "peak": PEAK_BF16_TFLOPS,
-            "unit": "TFLOP/s",
-            "frac": round(dq_exec / PEAK_BF16_TFLOPS, 4),
-            "traffic": None,
-            "note": "three executed products per launch (S, dP, dQ); one of them (dQ) is algorithmic",
-            "avg_ms": round(dq_avg, 4),
+            "algorithmic_bytes": 16 * bthd + 8 * B * H * T,
+            "note": "seven executed products per launch; five of them are algorithmic",
+            "avg_ms": round(bwd_avg, 4),
         }
     else:
+        # dominant kernel: the dK/dV kernel (4 products: S, dP, dV = P^T dO, dK = dS^T Q)
+        kv_avg = avg(kv_ms)
+        achieved = 4.0 * unit / (kv_avg * 1e-3) / 1e12
+        # dQ kernel from the stored dS: reads every dS tile once, K (once per 128-query block, from L2
+        # after the first), writes dQ fp32 once; algorithmic bytes = dS + K + dQ
+        dq_bytes = ws_bytes + 2 * bthd + 4 * bthd
+        dq_avg = avg(dq_ms)
         roofline = {
             "kernel": "backward dK/dV kernel with the dS store (mla::bwd_kernel<D, true>)",
             "bound": "mfma",
@@ -514,10 +519,8 @@ def main():
         "marked_ms_per_step": round(marked_ms, 4),
         "phases": {
             "fwd_ms_median": round(med(fwd_ms), 4), "computeD_ms_median": round(med(cd_ms), 4),
-            "bwd_ms_median": round(med(bwd_ms), 4), "bwd_dkdv_ms_median": round(med(kv_ms), 4),
-            "bwd_dq_ms_median": round(med(dq_ms), 4),
-            "bwd_recompute_ms_median": round(med(rc_bwd), 4), "bwd_recompute_dkdv_ms_median": round(med(rc_kv), 4),
-            "bwd_recompute_dq_ms_median": round(med(rc_dq), 4),
+            "bwd_ms_median": round(med(bwd_ms), 4), "bwd_dkdv_ms_median": med4(kv_ms), "bwd_dq_ms_median": med4(dq_ms),
+            "bwd_recompute_ms_median": round(med(r["rc_bwd"]), 4),
             "workspace_bytes": ws_bytes,
             "fwd_tflops": round(ff / (med(fwd_ms) * 1e-3) / 1e12, 2),
             "bwd_tflops": round(fb / (med(bwd_ms) * 1e-3) / 1e12, 2),
@@ -529,7 +532,7 @@ def main():
             "ms_per_step": round(rc_ms, 4),
             "tflops": round((ff + fb) / (rc_ms * 1e-3) / 1e12, 2),
             "pct_of_peak": round(100.0 * (ff + fb) / (rc_ms * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, 2),
-            "bwd_ms_median": round(med(rc_bwd), 4),
+            "bwd_ms_median": round(med(r["rc_bwd"]), 4),
         },
         "roofline": roofline,
     }

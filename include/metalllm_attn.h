@@ -109,8 +109,7 @@ int metalllmAttnBackwardWorkspaceSize(const AttentionParams* p, uint64_t* bytes)
  * flashAttentionBackward): the caller needs no zeroing pass and the dQ kernel no read of 4*B*M*N
  * bytes, 1.1 GB of HBM traffic less per step at B = NH = 16, M = 4096, D = 128. Its values equal
  * what flashAttentionBackward adds into a zeroed dQ up to fp32 summation order. The workspace
- * holds no state between calls, but one
- * workspace must not serve two calls at once. Returns METALLLM_ATTN_E_NULL / _E_ALIGN / _E_SIZE
+ * holds no state between calls, but one workspace must not serve two calls at once. Returns METALLLM_ATTN_E_NULL / _E_ALIGN / _E_SIZE
  * for a NULL, misaligned or too small workspace. At D = 64, and at D = 128 while B*NH*ceil(M/128) is
  * at most 512 (384 for M < 512), no dS is stored and the workspace is validated but not used:
  * it runs flashAttentionBackward's kernel writing dQ instead of adding into it (there the
@@ -118,8 +117,8 @@ int metalllmAttnBackwardWorkspaceSize(const AttentionParams* p, uint64_t* bytes)
  * flashAttentionBackward's into a zeroed dQ bit for bit.
  * An output may lie in an input's memory where the kernels allow it: dV in v's, and dQ in that of
  * q, v and dZ, at D = 128; dV in v's and dK in k's at D = 64 with M <= 256 (there in
- * flashAttentionBackward too). Such a call runs the
- * stored-dS kernels or the fused one at any number of pairs.
+ * flashAttentionBackward too). Such a call runs the stored-dS kernels or the fused one at any number
+ * of pairs.
  * No counterpart in the reference. */
 int flashAttentionBackwardWorkspace(const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
                                     const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
@@ -132,7 +131,7 @@ int flashAttentionBackwardWorkspace(const uint16_t* dZ, const float* d, const fl
  * with the dS tiles in a fixed per-device array of METALLLM_ATTN_NOALLOC_SCRATCH_BYTES (64 MiB,
  * held by every GPU the library runs on until the process ends) instead of a caller workspace.
  * Calls no hipMalloc/hipFree. D = 128 shapes whose metalllmAttnBackwardWorkspaceSize exceeds the
- * array return METALLLM_ATTN_E_SIZE (e.g. B = 4, NH = 12, M = 1024 needs 53.5 MB and fits; B = 8
+ * array return METALLLM_ATTN_E_SIZE, also those that would store no dS (e.g. B = 4, NH = 12, M = 1024 needs 53.5 MB and fits; B = 8
  * does not). D = 64 stores no dS tiles (see flashAttentionBackwardWorkspace) and accepts every
  * shape. All calls on one GPU share the array: calls that overlap on one GPU race. The first call
  * on a device looks up the array's address there. */
@@ -148,8 +147,9 @@ int flashAttentionBackwardNoAlloc(const uint16_t* dZ, const float* d, const floa
  * fp32 [N, N]. Products are computed with fp32 accumulation and rounded once to the destination
  * type: on hand-written kernels while N is a multiple of 64 and the product is small or fits no
  * 128-wide tile; larger ones run computeGradDx, computeGradDw and projBackwarddW on hand-written
- * kernels when B*M and N are multiples of 128, and the rest on rocBLAS gemm_ex. The "accumulate" kernels read their destination once and add to it, as
- * the reference's multiply_accumulate matmuls do; the caller zeroes those destinations first
+ * kernels when B*M and N are multiples of 128, and the rest on rocBLAS gemm_ex. The "accumulate"
+ * kernels read their destination once and add to it, as the reference's multiply_accumulate matmuls
+ * do; the caller zeroes those destinations first
  * (model.h:549-555). Validation: M, B, NH, D >= 1, N == NH*D a multiple of 8, tensors below 2^31
  * elements, non-NULL 16-byte aligned pointers. The first call on a device creates that device's
  * rocBLAS handle; computeGradDx/Dw keep a per-device buffer for the two-term bf16 split of dQ, and
@@ -325,8 +325,8 @@ int metalllmSublayerGraphDestroy(metalllmSublayerGraph* g);
  * entry points on `stream`: part 0 = dK/dV and part 1 = dQ recomputing the softmax
  * (flashAttentionBackward does the work of part 0 and part 1, in one launch, bit for bit the same);
  * part 2 = dK/dV storing dS into the workspace and part 3 = dQ from the stored dS
- * (flashAttentionBackwardWorkspace: likewise part 2 and part 3, two launches where dS is stored). Same validation and return
- * codes as those entry points (parts 0 and 1 ignore the workspace arguments); a part outside
+ * (flashAttentionBackwardWorkspace: likewise part 2 and part 3, two launches where dS is stored). Same
+ * validation and return codes as those entry points (parts 0 and 1 ignore the workspace arguments); a part outside
  * 0..3 returns METALLLM_ATTN_E_LAYOUT. Where the entry points run the fused short-sequence kernel,
  * parts 0 and 2 launch it (part 0 adds dQ, part 2 writes it) and parts 1 and 3 launch nothing. Where
  * the workspace entry point stores no dS, parts 2 and 3 launch parts 0's and 1's kernels, part 3

@@ -179,9 +179,10 @@ def flashAttentionBackwardNoAlloc(dZ, d, l, q, k, v, dQ, dK, dV, stream=None, pa
 
 def backward_part(part: int, dZ, d, l, q, k, v, dQ, dK, dV, stream=None, params: AttentionParams | None = None,
                   workspace=None):
-    """One kernel of the backward entry points (0: dK/dV, 1: dQ recomputing the softmax = the two
-    kernels of flashAttentionBackward; 2: dK/dV storing dS into `workspace`, 3: dQ from the stored
-    dS = flashAttentionBackwardWorkspace); the bench times them separately."""
+    """One half of a backward by itself (0: dK/dV, 1: dQ recomputing the softmax, added; 2 and 3: the
+    same of flashAttentionBackwardWorkspace, which stores dS into `workspace` in between or
+    recomputes): where the entry points run two kernels, those, which the bench times separately;
+    where they run one launch (backward_route), its halves, with the same results."""
     p = params or _shape(q)
     wp, wn = _ws(workspace)
     _check(_lib().metalllmAttnBackwardPart(part, _ptr(dZ), _ptr(d), _ptr(l), _ptr(q), _ptr(k), _ptr(v), _ptr(dQ),

@@ -2,9 +2,10 @@
 // (flashAttentionBackwardWorkspace) for callers that cannot allocate device memory (code under
 // HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). The dS tiles go into a
 // file-scope device array of METALLLM_ATTN_NOALLOC_SCRATCH_BYTES instead of a caller workspace;
-// shapes whose tiles do not fit are rejected. At D = 64 the workspace entry point stores no dS
-// tiles (the fused short-sequence kernel, or the recomputing kernels), so every D = 64 shape
-// fits. Every GPU the library runs on holds its own copy of the array until the process ends, and
+// shapes whose tiles would not fit are rejected, at D = 128 by their nominal size, also where the
+// workspace entry point stores none (few blocks: which kernels run then also depends on the buffers).
+// At D = 64 it never stores dS tiles (the fused short-sequence kernel, or the recomputing kernels), so
+// every D = 64 shape fits. Every GPU the library runs on holds its own copy of the array until the process ends, and
 // every call on one GPU shares it: calls that overlap on one GPU (different streams, or different
 // host threads) race. The kernels write every dS tile they read within one call, so the array
 // needs no clearing between calls.

@@ -145,7 +145,7 @@ __device__ __forceinline__ void products(Acc& acc, const u32x4 (&A)[2], const u3
     for (int j = 0; j < 2; ++j) acc.v[i][j] = mfma(A[i], B[j], acc.v[i][j]);
 }
 
-// Adds the 8 waves' tiles in wave order; put(row, column, four consecutive values) for each.
+// Adds the NW waves' tiles in wave order; put(row, column, four consecutive values) for each.
 template <int NW, class Put>
 __device__ __forceinline__ void reduce_tiles(const Lane& L, int tid, int wave, uint32_t smem, const Acc& acc, Put put) {
   // row p of a partial tile: 16 chunks of 4 floats, chunk c at c ^ (p & 15)
