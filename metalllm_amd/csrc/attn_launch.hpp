@@ -138,6 +138,7 @@ __host__ __device__ inline void decode_workgroup(int bid, int npairs, int nblk, 
 // Workgroups are dealt to the XCDs in turn and, inside an XCD, to its CUs in turn while they are
 // free: ids that differ by a multiple of kCus start on the same CU.
 constexpr int kCus = 256;
+static_assert((kCus & (kCus - 1)) == 0, "rows of kCus ids by masks (fwd_item_of)");
 
 __host__ __device__ inline bool backward_is_short(int T, int D, int pairs) {
   const int rounds = (pairs + kCus - 1) / kCus;
@@ -157,24 +158,25 @@ __host__ __device__ inline bool backward_is_short(int T, int D, int pairs) {
 // the list goes block by block, longest first, and its first W items snake over rows of one
 // workgroup per CU, so that the workgroups that share a CU have about the same work together. (Pair
 // by pair, the workgroups w, w + 256 and w + 512 of 12 pairs of T = 8192 all had blocks of the same
-// length and the CUs with the longest three took twice the mean: 204 us.)
+// length and the CUs with the longest three took twice the mean: 204 us.) Shifts for the groups of 8 and
+// the rows: the smallest calls wait for this arithmetic (one division is left).
 __host__ __device__ inline bool fwd_item_of(int bid, int grid, int k, int npairs, int nblk, int& pair, int& blk) {
-  const int G = ((npairs & 7) == 0 && (grid & 7) == 0) ? 8 : 1;
-  const int x = bid % G, W = grid / G, n = npairs / G * nblk;
-  int w = bid / G;
+  const int sh = ((npairs | grid) & 7) == 0 ? 3 : 0;  // 8 groups or one
+  const int x = bid & ((1 << sh) - 1), W = grid >> sh, n = (npairs >> sh) * nblk;
+  int w = bid >> sh;
   const bool few = n < 2 * W;
   if (few) {
-    const int row = kCus / G, r = w / row;
-    if (r & 1) {  // this row's ids in reverse
-      const int end = (r + 1) * row < W ? (r + 1) * row : W;
-      w = r * row + (end - 1 - w);
+    const int row = kCus >> sh, at = w & ~(row - 1);  // the row's first id
+    if (w & row) {                                    // every second row's ids in reverse
+      const int end = at + row < W ? at + row : W;
+      w = at + (end - 1 - w);
     }
   }
   const int m = k * W + ((k & 1) ? W - 1 - w : w);
   if (m >= n) return false;
-  const int per = few ? npairs / G : nblk;
+  const int per = few ? npairs >> sh : nblk;
   const int i = m / per, j = m - i * per;
-  pair = (few ? j : i) * G + x;
+  pair = ((few ? j : i) << sh) + x;
   blk = nblk - 1 - (few ? i : j);
   return true;
 }
