@@ -42,8 +42,9 @@ def S():
 
 @pytest.mark.parametrize("fused", [False, True])
 def test_forward_gemms(gpu, S, fused):
-    """fused: q_w, k_w, v_w are slices of one [3, C, C] buffer and q, k, v of one [3, R, C] buffer,
-    so computeQKV runs one strided-batched product; otherwise separate buffers and three."""
+    """fused: q_w, k_w, v_w are slices of one [3, C, C] buffer and q, k, v of one [3, R, C] buffer (a
+    larger computeQKV would run one strided-batched product, else three; here the tile kernel takes
+    either layout)."""
     import torch
     B, T, H, C = 2, 256, 12, 768
     R = B * T
@@ -77,14 +78,10 @@ def test_forward_gemms(gpu, S, fused):
 
 @pytest.mark.parametrize("B,T,H,C", [(2, 256, 12, 768), (1, 384, 3, 384), (1, 256, 4, 512), (1, 320, 5, 200)])
 def test_backward_gemms(gpu, S, B, T, H, C):
-    """R and C multiples of 128 run the hand-written computeGradDx and computeGradDw kernels (fp32
-    dQ split in registers), with 192-wide feature tiles where 192 divides C (768, 384) and 128-wide
-    ones otherwise (512); the last shape runs the library path on the split dQ. For computeGradDw,
-    R=512, C=768 gives 24 tiles of 128 x 192 with 8 dWq and 4 dKw/dVw row chunks each (384 items,
-    dealt to the XCDs in contiguous ranges), R=384, C=384 gives 72 (not a multiple of 8 per kind:
-    workgroup order) with dWq chunks of one 64-row step, and R=256, C=512 gives 16 tiles of 128 x
-    128; projBackwarddW (128-wide tiles) takes 144, 27 and 32 one-weight items. All are called
-    twice, so the second call accumulates into nonzero destinations."""
+    """The first three shapes run the 64 x 64 tile kernels (fp32 dQ split in registers; the 128-wide
+    ones, which take larger shapes, are in test_config4_full_size, test_config4_chain_at_config1_shape
+    and test_gpu_sublayer_wide.py); the last, C = 200, runs the library path on the split dQ. All are
+    called twice, so the second call accumulates into nonzero destinations."""
     import torch
     R = B * T
     X, (Wq, Wk, Wv, Wp) = inputs(R, C, 2)
