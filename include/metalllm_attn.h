@@ -89,8 +89,9 @@ int computeD(const uint16_t* dO, const uint16_t* O, float* D, const AttentionPar
  * into as in the reference: zero it first for the plain gradient); dK, dV = gradients (bf16).
  * One launch: dK/dV by key-block owners and dQ by query-block owners, each recomputing the
  * softmax tile it needs. For D = 64 and M = 128 to 256 (the reference's own shape), where B*NH fills
- * rounds of one pair per CU (nearly full ones, four at M = 128 and two at 192), a workgroup per (b, head) does both and keeps the dS tiles in LDS (dK,
- * dV bit-identical to the other form's, dQ equal up to fp32 summation order). */
+ * rounds of one pair per CU (nearly full ones, four at M = 128 and two at 192), a workgroup per
+ * (b, head) does both and keeps the dS tiles in LDS (dK, dV bit-identical to the other form's, dQ
+ * equal up to fp32 summation order). */
 int flashAttentionBackward(const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
                            const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
                            const AttentionParams* p, metalllm_stream_t stream);
@@ -109,9 +110,10 @@ int metalllmAttnBackwardWorkspaceSize(const AttentionParams* p, uint64_t* bytes)
  * flashAttentionBackward): the caller needs no zeroing pass and the dQ kernel no read of 4*B*M*N
  * bytes, 1.1 GB of HBM traffic less per step at B = NH = 16, M = 4096, D = 128. Its values equal
  * what flashAttentionBackward adds into a zeroed dQ up to fp32 summation order. The workspace
- * holds no state between calls, but one workspace must not serve two calls at once. Returns METALLLM_ATTN_E_NULL / _E_ALIGN / _E_SIZE
- * for a NULL, misaligned or too small workspace. At D = 64, and at D = 128 while B*NH*ceil(M/128) is
- * at most 512 (384 for M < 512), no dS is stored and the workspace is validated but not used:
+ * holds no state between calls, but one workspace must not serve two calls at once. Returns
+ * METALLLM_ATTN_E_NULL / _E_ALIGN / _E_SIZE for a NULL, misaligned or too small workspace. At D = 64,
+ * and at D = 128 while B*NH*ceil(M/128) is at most 512 (384 for M < 512), no dS is stored and the
+ * workspace is validated but not used:
  * it runs flashAttentionBackward's kernel writing dQ instead of adding into it (there the
  * recomputation in one launch is faster than the dS round trip's two), so dQ, dK and dV equal
  * flashAttentionBackward's into a zeroed dQ bit for bit.
@@ -131,10 +133,10 @@ int flashAttentionBackwardWorkspace(const uint16_t* dZ, const float* d, const fl
  * with the dS tiles in a fixed per-device array of METALLLM_ATTN_NOALLOC_SCRATCH_BYTES (64 MiB,
  * held by every GPU the library runs on until the process ends) instead of a caller workspace.
  * Calls no hipMalloc/hipFree. D = 128 shapes whose metalllmAttnBackwardWorkspaceSize exceeds the
- * array return METALLLM_ATTN_E_SIZE, also those that would store no dS (e.g. B = 4, NH = 12, M = 1024 needs 53.5 MB and fits; B = 8
- * does not). D = 64 stores no dS tiles (see flashAttentionBackwardWorkspace) and accepts every
- * shape. All calls on one GPU share the array: calls that overlap on one GPU race. The first call
- * on a device looks up the array's address there. */
+ * array return METALLLM_ATTN_E_SIZE, also those that would store no dS (e.g. B = 4, NH = 12, M = 1024
+ * needs 53.5 MB and fits; B = 8 does not). D = 64 stores no dS tiles (see
+ * flashAttentionBackwardWorkspace) and accepts every shape. All calls on one GPU share the array:
+ * calls that overlap on one GPU race. The first call on a device looks up the array's address there. */
 #define METALLLM_ATTN_NOALLOC_SCRATCH_BYTES (64ull << 20)
 int flashAttentionBackwardNoAlloc(const uint16_t* dZ, const float* d, const float* l, const uint16_t* q,
                                   const uint16_t* k, const uint16_t* v, float* dQ, uint16_t* dK, uint16_t* dV,
@@ -326,8 +328,8 @@ int metalllmSublayerGraphDestroy(metalllmSublayerGraph* g);
  * (flashAttentionBackward does the work of part 0 and part 1, in one launch, bit for bit the same);
  * part 2 = dK/dV storing dS into the workspace and part 3 = dQ from the stored dS
  * (flashAttentionBackwardWorkspace: likewise part 2 and part 3, two launches where dS is stored). Same
- * validation and return codes as those entry points (parts 0 and 1 ignore the workspace arguments); a part outside
- * 0..3 returns METALLLM_ATTN_E_LAYOUT. Where the entry points run the fused short-sequence kernel,
+ * validation and return codes as those entry points (parts 0 and 1 ignore the workspace arguments);
+ * a part outside 0..3 returns METALLLM_ATTN_E_LAYOUT. Where the entry points run the fused short-sequence kernel,
  * parts 0 and 2 launch it (part 0 adds dQ, part 2 writes it) and parts 1 and 3 launch nothing. Where
  * the workspace entry point stores no dS, parts 2 and 3 launch parts 0's and 1's kernels, part 3
  * writing dQ. */
